@@ -35,19 +35,8 @@
 // host and for later phases.  Each kernel exits at once when st->done is set,
 // so the host can queue many iterations ahead and poll rarely.  Inner
 // products and norms are accumulated in FP64 in both precisions.
-#include <hip/hip_ext.h>
-
 #include "nsx_kernels.h"
 
-// With timing on, a kernel is launched with its own start/stop events
-// (recorded by the dispatch itself, so the elapsed time is the kernel's)
-#define LAUNCH_TIMED(ev, q, kern, grid, blk, lds, s, ...)                                         \
-  do {                                                                                          \
-    if (ev)                                                                                     \
-      hipExtLaunchKernelGGL(kern, grid, blk, lds, s, (ev)[2 * (q)], (ev)[2 * (q) + 1], 0, __VA_ARGS__); \
-    else                                                                                        \
-      hipLaunchKernelGGL(kern, grid, blk, lds, s, __VA_ARGS__);                                 \
-  } while (0)
 
 #define FOR_EACH_CELL(g, c)                                                         \
   uint32_t beg_, end_;                                                              \
@@ -287,8 +276,9 @@ __global__ __launch_bounds__(NSX_BLOCK) void k_bicg_init_state(SolverState *st, 
   if (threadIdx.x == 0) {
     reset_state(st, eps, max_iters);
     st->mp_pass = 0;
-    st->m_stop = 0;
     st->m_iters = 0;
+    st->m_cyc = 0;
+    st->m_stall = 0;
     st->delta = delta;
     st->ureq[0] = st->ureq[1] = 0;
   }
@@ -2021,753 +2011,119 @@ int solver_blocks_per_cu(const Geo &g) {
   return best;
 }
 
-// ------------------------------------- CG with the vertical-mode preconditioner
-// (NSX_REFINE_MODAL; the tables and their meaning: nsx_modal.hip).  A
-// residual r (FP32, column-contiguous) goes to modal coefficients column by
-// column, rh_m = sum_k Phi[k][m] r(k+1); the lowest m0 go through one
-// V-cycle of the 2D aggregation multigrid, the others are divided by their
-// diagonal d_i + mu_m area_i; u = -Phi x (the operator is -(L (x) S + D (x)
-// T)).  Both transforms are GEMMs of the N0 columns against the mode table:
-// on the matrix cores (v_mfma_f32_16x16x4_f32, FP32 in and out) when the
-// columns have at most 128 slots, else on the vector units.
-
-// --- matrix-core transforms.  A wave forms 16 columns x all modes (or
-// interior layers): its lane (j, g) = (lane & 15, lane >> 4) holds float4s of
-// column c0 + j at interior layers (or modes) 16 t + 4 g .. +3, which are the
-// A operand of four MFMAs (k index 4 g + q of step (t, q)); the table's float4
-// for (t, tile, lane) holds the matching B operands, laid out by the host so
-// that one ds_read_b128 per lane fetches them.  The result D[i][j] of a 16 x
-// 16 tile sits in lane j + 16 (i / 4), register i % 4.  Layers and modes are
-// both padded to mp = 16 MT (zero rows and columns of the table).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ inline f32x4 mfma4(const float4 &a, const float4 &b, f32x4 c) {
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
-}
-
-// the transform kernels' blocks: 4 waves share one operand table in LDS
-constexpr int MODAL_TB = 256;
-
-// the operand table (64 MT^2 float4s) into LDS, every load issued before the
-// first store
-template <int MT>
-__device__ inline void lds_table(float4 *dst, const float4 *src) {
-  constexpr int n = 64 * MT * MT, U = (n + MODAL_TB - 1) / MODAL_TB;
-  float4 v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = threadIdx.x + u * MODAL_TB;
-    if (q < n) v[u] = src[q];
-  }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int q = threadIdx.x + u * MODAL_TB;
-    if (q < n) dst[q] = v[u];
-  }
-  __syncthreads();
-}
-
-// LDS written by some lanes of a wave, then read by others: ordered at the
-// wavefront's scope
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// the A operands of the forward transform: interior layers 16 t + 4 g .. +3 of
-// column c (slots one above; four-byte aligned, so one unaligned dwordx4
-// where all four are interior, single loads at the top, zero above nzi)
-template <int MT>
-__device__ inline void load_cols(const float *r, int NS, int N0, int nzi, int c, int gq, float4 (&a)[MT]) {
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int k = 16 * t + 4 * gq;
-    a[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c >= N0) continue;
-    const float *src = r + (size_t)c * NS + 1 + k;
-    if (k + 4 <= nzi) {
-      __builtin_memcpy(&a[t], src, sizeof(float4));
-    } else {
-      if (k < nzi) a[t].x = src[0];
-      if (k + 1 < nzi) a[t].y = src[1];
-      if (k + 2 < nzi) a[t].z = src[2];
-    }
-  }
-}
-
-template <int MT>
-__device__ inline void load_modes(const float *xh, int N0, int c, int gq, float4 (&a)[MT]) {
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    a[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (c < N0) a[t] = *(const float4 *)(xh + (size_t)c * (16 * MT) + 16 * t + 4 * gq);
-  }
-}
-
-// the same with the 16 multigrid modes formed here: the V-cycle's last step,
-// the level-0 post-smoothing x = y + omega (b - A y) / d with y = omega z +
-// x_1(agg) at the column and its neighbours (the arithmetic of k_mg_up<1>),
-// for modes 4 g .. +3; the other modes from xh
-__device__ inline float4 ld4f(const float *p) { return *(const float4 *)p; }
-
-template <int MT>
-__device__ inline void load_modes_v0(const ModalDev &M, int N0, int c, int gq, float4 (&a)[MT]) {
-  load_modes<MT>(M.xh, N0, c, gq, a);
-  if (c >= N0) return;
-  const ModalLevelDev &F = M.lev[0];
-  const float om = NSX_MODAL_OMEGA;
-  const float *z = M.z[0], *b = M.b[0], *x1 = M.x[1];
-  const int m = 4 * gq;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int e = F.ptr[c]; e < F.ptr[c + 1]; ++e) {
-    const float4 zj = ld4f(z + (size_t)F.col[e] * 16 + m), xj = ld4f(x1 + (size_t)F.eagg[e] * 16 + m);
-    const float w = F.w[e];
-    acc[0] = fmaf(w, fmaf(om, zj.x, xj.x), acc[0]);
-    acc[1] = fmaf(w, fmaf(om, zj.y, xj.y), acc[1]);
-    acc[2] = fmaf(w, fmaf(om, zj.z, xj.z), acc[2]);
-    acc[3] = fmaf(w, fmaf(om, zj.w, xj.w), acc[3]);
-  }
-  const float4 zc = ld4f(z + (size_t)c * 16 + m), bc = ld4f(b + (size_t)c * 16 + m),
-               xc = ld4f(x1 + (size_t)F.agg[c] * 16 + m);
-  const float zv[4] = {zc.x, zc.y, zc.z, zc.w}, bv[4] = {bc.x, bc.y, bc.z, bc.w}, xv[4] = {xc.x, xc.y, xc.z, xc.w};
-  const float dgc = F.diag[c], arc = F.area[c];
-  float o[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float di = dgc + M.mu[m + k] * arc;
-    const float yi = fmaf(om, zv[k], xv[k]);
-    const float ay = fmaf(di, yi, -acc[k]);
-    o[k] = yi + om * (bv[k] - ay) / di;
-  }
-  a[0] = make_float4(o[0], o[1], o[2], o[3]);
-}
-
-// MT = mp / 16.  Two blocks of 4 waves a CU; a wave with more than one tile
-// loads its next tile's operands before it forms the current one.  STAGE:
-// the wave's 16 rows of xh (one contiguous stretch) are assembled in LDS and
-// leave as aligned float4s; the low modes' entries written there are
-// overwritten by the V-cycle's last prolongation.  The diagonal scaling
-// multiplies by v_rcp_f32 of d (a fixed diagonal: the preconditioner stays
-// symmetric).
-template <int MT, bool STAGE>
-__global__ __launch_bounds__(MODAL_TB, 1) void k_modal_fwd_mfma(Geo g, ModalDev M, const float *r,
-                                                                 const SolverState *st) {
-  if (st->m_stop) return;
-  extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
-  float4 *tab = reinterpret_cast<float4 *>(nsx_dyn_lds);
-  const int m0 = M.m0, nzi = M.nzi;
-  constexpr int MP = 16 * MT;
-  lds_table<MT>(tab, M.tfwd);
-  const int lane = threadIdx.x & 63, j = lane & 15, gq = lane >> 4;
-  float *stg = reinterpret_cast<float *>(tab + 64 * MT * MT) + (size_t)(threadIdx.x >> 6) * 16 * MP;
-  const int ntile = (g.N0 + 15) >> 4, stride = gridDim.x * (MODAL_TB / 64);
-  int tile = blockIdx.x * (MODAL_TB / 64) + (threadIdx.x >> 6);
-  float4 a[MT], an[MT];
-  load_cols<MT>(r, g.NS, g.N0, nzi, tile * 16 + j, gq, a);
-  for (; tile < ntile; tile += stride) {
-    if (tile + stride < ntile) load_cols<MT>(r, g.NS, g.N0, nzi, (tile + stride) * 16 + j, gq, an);
-    const int c0 = tile * 16;
-    f32x4 acc[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // one layer tile at a time: the scheduler keeps a step's table operands
-    // (MT float4s) in flight, not the whole table
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma4(a[t], tab[(t * MT + mt) * 64 + lane], acc[mt]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    float dg[4], ar[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = min(c0 + 4 * gq + q, g.N0 - 1);
-      dg[q] = M.lev[0].diag[c];
-      ar[q] = M.lev[0].area[c];
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m = 16 * mt + j;
-      const float mum = M.mu[m];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c = c0 + 4 * gq + q;
-        const float v = acc[mt][q], x = v * __builtin_amdgcn_rcpf(dg[q] + mum * ar[q]);
-        if (STAGE) stg[(4 * gq + q) * MP + m] = x;
-        if (c >= g.N0) continue;
-        if (m < m0) {
-          M.b[0][(size_t)c * m0 + m] = v;
-          M.z[0][(size_t)c * m0 + m] = x;
-        } else if (!STAGE) {
-          M.xh[(size_t)c * MP + m] = x;
-        }
-      }
-    }
-    if (STAGE) {
-      wave_lds_sync();
-      const int nf = min(16, g.N0 - c0) * MP;
-      float *xt = M.xh + (size_t)c0 * MP;
-      for (int o = 4 * lane; o < nf; o += 256) *(float4 *)(xt + o) = *(const float4 *)(stg + o);
-      wave_lds_sync();
-    }
-#pragma unroll
-    for (int t = 0; t < MT; ++t) a[t] = an[t];
-  }
-}
-
-// u = -Phi x from the modal coefficients xh (N0 x mp) at the interior layers,
-// zero at the other slots; partial sums of <r, u>.  STAGE: the wave's 16
-// columns (one contiguous stretch of u) are assembled in LDS and leave, with
-// r read beside them for <r, u>, as aligned float4s (else each lane stores
-// its outputs where they go, in 64-byte runs that straddle two segments).
-template <int MT, bool STAGE, bool V0>
-__global__ __launch_bounds__(MODAL_TB, 1) void k_modal_bwd_mfma(Geo g, ModalDev M, const float *r, float *u,
-                                                                 double *P, const SolverState *st) {
-  if (st->m_stop) return;
-  extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
-  float4 *tab = reinterpret_cast<float4 *>(nsx_dyn_lds);
-  const int nzi = M.nzi, NS = g.NS;
-  lds_table<MT>(tab, M.tbwd);
-  const int lane = threadIdx.x & 63, j = lane & 15, gq = lane >> 4;
-  float *stg = reinterpret_cast<float *>(tab + 64 * MT * MT) + (size_t)(threadIdx.x >> 6) * 16 * NS;
-  const int ntile = (g.N0 + 15) >> 4, stride = gridDim.x * (MODAL_TB / 64);
-  int tile = blockIdx.x * (MODAL_TB / 64) + (threadIdx.x >> 6);
-  double acc2[1] = {0.0};
-  float4 a[MT], an[MT];
-  if (V0)
-    load_modes_v0<MT>(M, g.N0, tile * 16 + j, gq, a);
-  else
-    load_modes<MT>(M.xh, g.N0, tile * 16 + j, gq, a);
-  for (; tile < ntile; tile += stride) {
-    if (tile + stride < ntile) {
-      if (V0)
-        load_modes_v0<MT>(M, g.N0, (tile + stride) * 16 + j, gq, an);
-      else
-        load_modes<MT>(M.xh, g.N0, (tile + stride) * 16 + j, gq, an);
-    }
-    const int c0 = tile * 16;
-    f32x4 acc[MT];
-#pragma unroll
-    for (int nt = 0; nt < MT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-#pragma unroll
-      for (int nt = 0; nt < MT; ++nt) acc[nt] = mfma4(a[t], tab[(t * MT + nt) * 64 + lane], acc[nt]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    const int nout = NS - nzi;  // slot 0 and nzi + 1 .. NS - 1
-    if (STAGE) {
-      for (int q = lane; q < 16 * nout; q += 64) {
-        const int cl = q / nout, o = q - cl * nout;
-        stg[cl * NS + (o == 0 ? 0 : nzi + o)] = 0.f;
-      }
-#pragma unroll
-      for (int nt = 0; nt < MT; ++nt) {
-        const int k = 16 * nt + j;
-        if (k >= nzi) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) stg[(4 * gq + q) * NS + k + 1] = 0.f - acc[nt][q];
-      }
-      wave_lds_sync();
-      const int ncol = min(16, g.N0 - c0), nf = ncol * NS;
-      float *ut = u + (size_t)c0 * NS;
-      const float *rt = r + (size_t)c0 * NS;
-      for (int o = 4 * lane; o < nf; o += 256) {
-        const float4 uv = *(const float4 *)(stg + o);
-        const float4 rv = *(const float4 *)(rt + o);
-        *(float4 *)(ut + o) = uv;
-        const int s0 = o % NS;  // NS is a multiple of 4: the float4 stays in one column
-        const float uu[4] = {uv.x, uv.y, uv.z, uv.w}, rr[4] = {rv.x, rv.y, rv.z, rv.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (s0 + q >= 1 && s0 + q <= nzi) acc2[0] += (double)rr[q] * (double)uu[q];
-      }
-      wave_lds_sync();
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < MT; ++nt) {
-        const int k = 16 * nt + j;
-        if (k >= nzi) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int c = c0 + 4 * gq + q;
-          if (c >= g.N0) continue;
-          const size_t sl = (size_t)c * NS + k + 1;
-          const float uv = 0.f - acc[nt][q];
-          u[sl] = uv;
-          acc2[0] += (double)r[sl] * (double)uv;
-        }
-      }
-      for (int q = lane; q < 16 * nout; q += 64) {
-        const int c = c0 + q / nout, o = q % nout;
-        if (c < g.N0) u[(size_t)c * NS + (o == 0 ? 0 : nzi + o)] = 0.f;
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < MT; ++t) a[t] = an[t];
-  }
-  write_partials<1, MODAL_TB>(acc2, P);
-}
-
-// --- vector-unit transforms for columns of more than 128 interior layers
-constexpr int MODAL_COLS = 32;  // columns a block transforms together
-constexpr int MODAL_CSTR = 36;  // LDS row stride of the column tile (float4-aligned, spreads the banks)
-
-__device__ inline bool modal_lds_fits(const ModalDev &M) {
-  return (size_t)M.nzp * M.nzp + (size_t)MODAL_CSTR * M.nzp <= 16384;
-}
-static size_t modal_lds(const ModalDev &M) {
-  const size_t t = (size_t)M.nzp * M.nzp + (size_t)MODAL_CSTR * M.nzp;
-  return (t <= 16384 ? t : (size_t)MODAL_CSTR * M.nzp) * sizeof(float);
-}
-
-// out[c][j] = sum_k tab[k][j] in[k][c] for the block's MODAL_COLS columns: a
-// thread forms a 4 x 4 tile (4 columns, 4 of j) from a float4 of the table
-// and a float4 of the column tile per k (tab: nzp x nzp row-major, in LDS or
-// global; tile: [k][MODAL_CSTR] in LDS); f(c, j, value) stores
-template <class F>
-__device__ inline void modal_tiles(const float *tab, const float *tile, int nzp, int nk, F &&f) {
-  const int nq = nzp / 4, nt = (MODAL_COLS / 4) * nq;
-  for (int q = threadIdx.x; q < nt; q += NSX_BLOCK) {
-    const int cq = q / nq, jq = q - cq * nq;
-    float a[4][4] = {};
-    for (int k = 0; k < nk; ++k) {
-      const float4 t = *(const float4 *)(tab + (size_t)k * nzp + 4 * jq);
-      const float4 x = *(const float4 *)(tile + (size_t)k * MODAL_CSTR + 4 * cq);
-      const float tv[4] = {t.x, t.y, t.z, t.w}, xv[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) a[cc][jj] = fmaf(tv[jj], xv[cc], a[cc][jj]);
-    }
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) f(4 * cq + cc, 4 * jq + jj, a[cc][jj]);
-  }
-}
-
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_fwd_vec(Geo g, ModalDev M, const float *r,
-                                                              const SolverState *st) {
-  if (st->m_stop) return;
-  extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
-  float *lds = reinterpret_cast<float *>(nsx_dyn_lds);
-  const int nzp = M.nzp, nzi = M.nzi, m0 = M.m0, MP = M.mp;
-  const bool in_lds = modal_lds_fits(M);
-  const float *ph = in_lds ? lds : M.phi;
-  float *rc = in_lds ? lds + (size_t)nzp * nzp : lds;
-  if (in_lds)
-    for (int q = threadIdx.x; q < nzp * nzp; q += NSX_BLOCK) lds[q] = M.phi[q];
-  const int ngrp = (g.N0 + MODAL_COLS - 1) / MODAL_COLS;
-  for (int grp = blockIdx.x; grp < ngrp; grp += gridDim.x) {
-    __syncthreads();
-    const int c0 = grp * MODAL_COLS;
-    for (int q = threadIdx.x; q < MODAL_COLS * nzp; q += NSX_BLOCK) {
-      const int c = q / nzp, k = q - c * nzp, i = c0 + c;
-      rc[(size_t)k * MODAL_CSTR + c] = (i < g.N0 && k < nzi) ? r[(size_t)i * g.NS + k + 1] : 0.f;
-    }
-    __syncthreads();
-    modal_tiles(ph, rc, nzp, nzi, [&](int c, int m, float v) {
-      const int i = c0 + c;
-      if (i >= g.N0 || m >= nzi) return;
-      const float d = M.lev[0].diag[i] + M.mu[m] * M.lev[0].area[i];
-      if (m < m0) {
-        M.b[0][(size_t)i * m0 + m] = v;
-        M.z[0][(size_t)i * m0 + m] = v / d;
-      } else {
-        M.xh[(size_t)i * MP + m] = v / d;
-      }
-    });
-  }
-}
-
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_bwd_vec(Geo g, ModalDev M, const float *r, float *u, double *P,
-                                                              const SolverState *st) {
-  if (st->m_stop) return;
-  extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
-  float *lds = reinterpret_cast<float *>(nsx_dyn_lds);
-  const int nzp = M.nzp, nzi = M.nzi, MP = M.mp;
-  const bool in_lds = modal_lds_fits(M);
-  const float *pt = in_lds ? lds : M.phiT;
-  float *xc = in_lds ? lds + (size_t)nzp * nzp : lds;
-  if (in_lds)
-    for (int q = threadIdx.x; q < nzp * nzp; q += NSX_BLOCK) lds[q] = M.phiT[q];
-  double acc[1] = {0.0};
-  const int ngrp = (g.N0 + MODAL_COLS - 1) / MODAL_COLS;
-  for (int grp = blockIdx.x; grp < ngrp; grp += gridDim.x) {
-    __syncthreads();
-    const int c0 = grp * MODAL_COLS;
-    for (int q = threadIdx.x; q < MODAL_COLS * nzp; q += NSX_BLOCK) {
-      const int c = q / nzp, m = q - c * nzp, i = c0 + c;
-      xc[(size_t)m * MODAL_CSTR + c] = (i < g.N0 && m < nzi) ? M.xh[(size_t)i * MP + m] : 0.f;
-    }
-    __syncthreads();
-    modal_tiles(pt, xc, nzp, nzi, [&](int c, int k, float v) {
-      const int i = c0 + c;
-      if (i >= g.N0 || k >= nzi) return;
-      const size_t s = (size_t)i * g.NS + k + 1;
-      u[s] = 0.f - v;
-      acc[0] += (double)r[s] * (double)(0.f - v);
-    });
-  }
-  // the slots outside the interior layers
-  const uint32_t nout = (uint32_t)(g.NS - nzi);
-  for (uint32_t t = blockIdx.x * NSX_BLOCK + threadIdx.x; t < (uint32_t)g.N0 * nout; t += gridDim.x * NSX_BLOCK) {
-    const uint32_t i = t / nout, j = t - i * nout;
-    const int k = j == 0 ? 0 : nzi + (int)j;
-    u[(size_t)i * g.NS + k] = 0.f;
-  }
-  write_partials<1>(acc, P);
-}
-
-// --- the batched 2D V-cycle on n_l x m0 arrays (node-major, mode fastest):
-// the operator of mode m at level l is d_i(m) - W, d_i(m) = diag_i + mu_m
-// area_i.  One damped Jacobi sweep from zero before the coarse correction
-// (x = omega z, z = b / d, written by the producer of b) and one after it; the
-// restriction forms the residual of the first where it needs it, and the
-// post-smoothing forms the prolonged y = omega z + P x_c at the node and its
-// neighbours: one launch per level each way.  Rows with many entries are
-// split over S slices of lanes (lane m + 16 s), summed by shuffles in a fixed
-// order.
-constexpr float MG_OMEGA = NSX_MODAL_OMEGA;
-
-template <int S>
-__device__ inline float slice_sum(float v) {
-  if (S >= 2) v += __shfl_xor(v, 16, 64);
-  if (S >= 4) v += __shfl_xor(v, 32, 64);
-  return v;
-}
-
-// b_c[J] = sum over the children i of J of (b - A x)_i with x = omega z:
-// (1 - omega) sum_i b_i + omega sum_j RW[J][j] z_j (RW = R W, the weights of
-// the children summed per fine neighbour), one CSR over the fine nodes with
-// a coefficient on b and one on z; z_c = b_c / d_J.  A wave per J.
-__global__ __launch_bounds__(NSX_BLOCK) void k_mg_down(ModalLevelDev C, const float *mu, int m0, const float *bf,
-                                                        const float *zf, float *bc, float *zc, const SolverState *st) {
-  if (st->m_stop) return;
-  const uint32_t t = blockIdx.x * NSX_BLOCK + threadIdx.x;
-  const int J = (int)(t >> 6), m = (int)(t & 15), sl = (int)((t >> 4) & 3);
-  if (J >= C.n) return;  // whole waves
-  float v = 0.f;
-  if (m < m0) {
-    for (int e = C.dptr[J] + sl; e < C.dptr[J + 1]; e += 4) {
-      const size_t q = (size_t)C.dcol[e] * m0 + m;
-      v = fmaf(C.db[e], bf[q], fmaf(C.dz[e], zf[q], v));
-    }
-  }
-  v = slice_sum<4>(v);
-  if (sl == 0 && m < m0) {
-    bc[(size_t)J * m0 + m] = v;
-    zc[(size_t)J * m0 + m] = v / (C.diag[J] + mu[m] * C.area[J]);
-  }
-}
-
-// x = C^-1 b on the coarsest level, C^-1 laid out [J][K][m]: a block per J,
-// 16 slices of K
-__global__ __launch_bounds__(NSX_BLOCK) void k_mg_coarse(int nc, int m0, const float *cinvT, const float *b, float *x,
-                                                          int ostride, const SolverState *st) {
-  if (st->m_stop) return;
-  __shared__ float sh[NSX_BLOCK / 64][16];
-  const int J = blockIdx.x, m = threadIdx.x & 15, sl = threadIdx.x >> 4;
-  float v = 0.f;
-  if (m < m0) {
-    const float *row = cinvT + (size_t)J * nc * m0 + m;
-    for (int K = sl; K < nc; K += NSX_BLOCK / 16) v = fmaf(row[(size_t)K * m0], b[(size_t)K * m0 + m], v);
-  }
-  v = slice_sum<4>(v);
-  if ((threadIdx.x & 63) < 16) sh[threadIdx.x >> 6][m] = v;
-  __syncthreads();
-  if (threadIdx.x < 16 && m < m0) {
-    float s = 0.f;
-    for (int w = 0; w < NSX_BLOCK / 64; ++w) s += sh[w][m];
-    x[(size_t)J * ostride + m] = s;
-  }
-}
-
-// x = y + omega (b - A y) / d with y = omega z + x_c(agg) at the node and its
-// neighbours; S slices per row (S = 4: a wave per row)
-template <int S>
-__global__ __launch_bounds__(NSX_BLOCK) void k_mg_up(ModalLevelDev F, const float *mu, int m0, const float *xc,
-                                                      const float *bf, const float *zf, float *xf, int ostride,
-                                                      const SolverState *st) {
-  if (st->m_stop) return;
-  const uint32_t t = blockIdx.x * NSX_BLOCK + threadIdx.x;
-  const int m = (int)(t & 15), sl = (int)((t >> 4) & (S - 1));
-  const uint32_t i = t / (16 * S);
-  if (S > 1 && i >= (uint32_t)F.n) return;  // whole waves
-  const bool act = i < (uint32_t)F.n && m < m0;
-  float acc = 0.f;
-  if (act)
-    for (int e = F.ptr[i] + sl; e < F.ptr[i + 1]; e += S)
-      acc = fmaf(F.w[e], fmaf(MG_OMEGA, zf[(size_t)F.col[e] * m0 + m], xc[(size_t)F.eagg[e] * m0 + m]), acc);
-  acc = slice_sum<S>(acc);
-  if (act && sl == 0) {
-    const size_t q = (size_t)i * m0 + m;
-    const float di = F.diag[i] + mu[m] * F.area[i];
-    const float yi = fmaf(MG_OMEGA, zf[q], xc[(size_t)F.agg[i] * m0 + m]);
-    const float ay = fmaf(di, yi, -acc);
-    xf[(size_t)i * ostride + m] = yi + MG_OMEGA * (bf[q] - ay) / di;
-  }
-}
-
-// (ev: null, or a start/stop pair the dispatch records)
-// the backward transform forms the V-cycle's level-0 post-smoothing where it
-// runs on the matrix cores with 16 multigrid modes and the V-cycle has a
-// level below the columns
-static bool modal_fused_v0(const ModalDev &M) { return M.mt <= 8 && M.m0 == 16 && M.nlev >= 2; }
-
-// staged kernels past 64 KB of LDS: the kernel's limit raised once (false
-// when the device does not allow it)
-static bool lds_allow(const void *kern, size_t bytes, int optin) {
-  if (bytes <= 65536) return true;
-  if (bytes > (size_t)optin) return false;
-  return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
-}
-
-template <int MT>
-static void launch_transforms_t(const Geo &g, hipStream_t s, const ModalDev &M, const float *r, float *u, double *P,
-                                const SolverState *st, bool fwd, hipEvent_t *ev) {
-  const size_t lds = (size_t)MT * MT * 64 * sizeof(float4);
-  if (fwd) {
-    // the staged forward transform where table and staging fit the LDS a
-    // block may have
-    const size_t fstage = (size_t)(MODAL_TB / 64) * 16 * (16 * MT) * sizeof(float);
-    static const bool fok =
-        lds_allow(reinterpret_cast<const void *>(&k_modal_fwd_mfma<MT, true>), lds + fstage, M.lds_optin);
-    if (fok)
-      LAUNCH_TIMED(ev, 0, (k_modal_fwd_mfma<MT, true>), dim3(M.agrid), dim3(MODAL_TB), lds + fstage, s, g, M, r, st);
-    else
-      LAUNCH_TIMED(ev, 0, (k_modal_fwd_mfma<MT, false>), dim3(M.agrid), dim3(MODAL_TB), lds, s, g, M, r, st);
-    return;
-  }
-  // the staged backward transform where table and staging fit the LDS a
-  // block may have; it forms the level-0 post-smoothing itself where the
-  // V-cycle left it out (modal_fused_v0)
-  const size_t stage = (size_t)(MODAL_TB / 64) * 16 * g.NS * sizeof(float);
-  const bool v0 = modal_fused_v0(M);
-  static size_t allowed = 65536;  // the staged kernels' LDS limit as set so far
-  if (lds + stage > allowed &&
-      lds_allow(reinterpret_cast<const void *>(&k_modal_bwd_mfma<MT, true, false>), lds + stage, M.lds_optin) &&
-      lds_allow(reinterpret_cast<const void *>(&k_modal_bwd_mfma<MT, true, true>), lds + stage, M.lds_optin))
-    allowed = lds + stage;
-  if (lds + stage <= allowed) {
-    if (v0)
-      LAUNCH_TIMED(ev, 0, (k_modal_bwd_mfma<MT, true, true>), dim3(M.agrid), dim3(MODAL_TB), lds + stage, s, g, M, r,
-                   u, P, st);
-    else
-      LAUNCH_TIMED(ev, 0, (k_modal_bwd_mfma<MT, true, false>), dim3(M.agrid), dim3(MODAL_TB), lds + stage, s, g, M, r,
-                   u, P, st);
-  } else {
-    if (v0)
-      LAUNCH_TIMED(ev, 0, (k_modal_bwd_mfma<MT, false, true>), dim3(M.agrid), dim3(MODAL_TB), lds, s, g, M, r, u, P,
-                   st);
-    else
-      LAUNCH_TIMED(ev, 0, (k_modal_bwd_mfma<MT, false, false>), dim3(M.agrid), dim3(MODAL_TB), lds, s, g, M, r, u, P,
-                   st);
-  }
-}
-
-// the matrix-core kernels take at most 128 interior layers (mp / 16 <= 8);
-// above, the vector units
-static void launch_transform(const Geo &g, hipStream_t s, const ModalDev &M, const float *r, float *u, double *P,
-                             const SolverState *st, bool fwd, hipEvent_t *ev) {
-  switch (M.mt) {
-    case 1: return launch_transforms_t<1>(g, s, M, r, u, P, st, fwd, ev);
-    case 2: return launch_transforms_t<2>(g, s, M, r, u, P, st, fwd, ev);
-    case 3: return launch_transforms_t<3>(g, s, M, r, u, P, st, fwd, ev);
-    case 4: return launch_transforms_t<4>(g, s, M, r, u, P, st, fwd, ev);
-    case 5: return launch_transforms_t<5>(g, s, M, r, u, P, st, fwd, ev);
-    case 6: return launch_transforms_t<6>(g, s, M, r, u, P, st, fwd, ev);
-    case 7: return launch_transforms_t<7>(g, s, M, r, u, P, st, fwd, ev);
-    case 8: return launch_transforms_t<8>(g, s, M, r, u, P, st, fwd, ev);
-    default: break;
-  }
-  const size_t lds = modal_lds(M);
-  if (fwd)
-    LAUNCH_TIMED(ev, 0, k_modal_fwd_vec, dim3(M.agrid), dim3(NSX_BLOCK), lds, s, g, M, r, st);
-  else
-    LAUNCH_TIMED(ev, 0, k_modal_bwd_vec, dim3(M.agrid), dim3(NSX_BLOCK), lds, s, g, M, r, u, P, st);
-}
-
-int launch_modal_apply(const Geo &g, hipStream_t s, const ModalDev &M, const float *r, float *u, Partials part,
-                       const SolverState *st, hipEvent_t *ev) {
-  const dim3 blk(NSX_BLOCK);
-  launch_transform(g, s, M, r, u, part.a, st, true, ev);
-  if (ev) (void)hipEventRecord(ev[2], s);
-  const int m0 = M.m0, L = M.nlev;
-  auto grid = [](size_t threads) { return dim3((unsigned)((threads + NSX_BLOCK - 1) / NSX_BLOCK)); };
-  for (int l = 0; l + 1 < L; ++l)
-    hipLaunchKernelGGL(k_mg_down, grid((size_t)M.lev[l + 1].n * 64), blk, 0, s, M.lev[l + 1], M.mu, m0, M.b[l],
-                       M.z[l], M.b[l + 1], M.z[l + 1], st);
-  // the coarsest solve and the last prolongation write the low modes into xh
-  hipLaunchKernelGGL(k_mg_coarse, dim3(M.nc), blk, 0, s, M.nc, m0, M.cinv, M.b[L - 1], L == 1 ? M.xh : M.x[L - 1],
-                     L == 1 ? M.mp : m0, st);
-  for (int l = L - 2; l >= (modal_fused_v0(M) ? 1 : 0); --l) {
-    float *out = l == 0 ? M.xh : M.x[l];
-    const int os = l == 0 ? M.mp : m0;
-    if (l == 0)
-      hipLaunchKernelGGL(k_mg_up<1>, grid((size_t)M.lev[l].n * 16), blk, 0, s, M.lev[l], M.mu, m0, M.x[l + 1],
-                         M.b[l], M.z[l], out, os, st);
-    else
-      hipLaunchKernelGGL(k_mg_up<4>, grid((size_t)M.lev[l].n * 64), blk, 0, s, M.lev[l], M.mu, m0, M.x[l + 1],
-                         M.b[l], M.z[l], out, os, st);
-  }
-  if (ev) (void)hipEventRecord(ev[3], s);
-  launch_transform(g, s, M, r, u, part.a, st, false, ev ? ev + 4 : nullptr);
-  return (int)hipGetLastError();
-}
-
-// p_out = u + beta p_in at the seven points, w = A p_out, <p, w>
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_spmv(Geo g, const float *u, const float *pin, float *pout,
-                                                           float *w, Partials P, SolverState *st, int first,
-                                                           uint32_t na) {
-  if (st->done || st->m_stop) return;
-  double t[1];
-  reduce_partials<1>(P.a, na, t);
-  const double rho = t[0];
-  // every block forms the same rho, so all return together
-  if (!first && fabs(rho) < NSX_MODAL_DROP * fabs(st->m_rho0)) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->m_stop = 1;
-    return;
-  }
-  const double beta = first ? 0.0 : rho / st->m_rho_prev;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->m_rho = rho;
-    if (first) st->m_rho0 = rho;
-  }
-  float *lvw = load_levels<float>(g);
-  for (int k = threadIdx.x; k < g.NS; k += NSX_BLOCK) lvw[2 * g.NS + k] = 1.f / lvw[k];
-  __syncthreads();
-  const float *lv = lvw;
-  double acc[1] = {0.0};
-  for_each_quad_gathered(
-      g, u, pin, (float)beta, first != 0, [&](size_t) {},
-      [&](int, int k0, size_t s0, const Col<float> &C, const float(&fc)[4], float fm, float fp,
-          const float(&f0)[4], const float(&f1)[4], const float(&f2)[4]) {
-        float qv[5], wo[4], po[4];
-        quot5_r(C, lv, g.NS, k0, qv);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const Row1<float> R = row_of(g, lv, C, qv, k0, v);
-          const float wv = apply_row(g, R, k0, v, fc, fm, fp, f0[v], f1[v], f2[v]);
-          wo[v] = R.in ? wv : 0.f;
-          po[v] = R.in ? fc[v] : 0.f;
-          if (R.in) acc[0] += (double)fc[v] * (double)wv;
-        }
-        st4(pout + s0, po);
-        st4(w + s0, wo);
-      });
-  write_partials<1>(acc, P.b);
-}
-
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_update(Geo g, const float *p, const float *w, float *e, float *r,
-                                                             Partials P, SolverState *st) {
-  if (st->done || st->m_stop) return;
-  double t[1];
-  reduce_partials<1>(P.b, gridDim.x, t);
-  const float alpha = (float)(st->m_rho / t[0]);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->m_rho_prev = st->m_rho;
-    st->m_iters += 1;
-  }
-  for_each_quad(g, [&](int, int, size_t s0) {
-    float pp[4], ww[4], ee[4], rr[4];
-    ld4(p + s0, pp);
-    ld4(w + s0, ww);
-    ld4(e + s0, ee);
-    ld4(r + s0, rr);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      ee[v] = fmaf(alpha, pp[v], ee[v]);
-      rr[v] = fmaf(-alpha, ww[v], rr[v]);
-    }
-    st4(e + s0, ee);
-    st4(r + s0, rr);
-  });
-}
-
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_true(Geo g, const double *rhs, const double *x, const float *e,
-                                                           float *r, Partials P, SolverState *st) {
+// ------------------------------------- the vertical-mode solve's residual
+// (NSX_REFINE_MODAL, nsx_modal_dev.hip)
+// r = b - A x in FP64 (zero outside the interior layers) and the partial sums
+// |r|^2, |r|_1, sum x Vol, four layers a thread with the neighbour window of
+// the BiCGSTAB's products
+__global__ __launch_bounds__(NSX_BLOCK) void k_modal_true(Geo g, const double *rhs, const double *x, double *r,
+                                                           Partials P, const SolverState *st) {
   if (st->done) return;
   const double avec = st->avec;
+  const double *lv = load_levels<double>(g);
   double acc[3] = {0.0, 0.0, 0.0};
-  FOR_EACH_CELL(g, c) {
-    int i, k;
-    cell_of(g, c, i, k);
-    double res, xs;
-    true_residual(g, rhs, x, avec, i, k, [&](size_t q, bool) { return e[q]; }, res, xs);
-    r[(size_t)i * g.NS + k] = (float)res;
-    acc[0] += res * res;
-    acc[1] += fabs(res);
-    acc[2] += xs * (g.area[i] * g.dsig[k]);
-  }
+  double bb[4];
+  for_each_quad_gathered(
+      g, x, x, 0.0, true, [&](size_t s0) { ld4(rhs + s0, bb); },
+      [&](int, int k0, size_t s0, const Col<double> &C, const double(&fc)[4], double fm, double fp,
+          const double(&f0)[4], const double(&f1)[4], const double(&f2)[4]) {
+        double qv[5], ro[4];
+        quot5(C, lv, k0, qv);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const Row1<double> R = row_of(g, lv, C, qv, k0, u);
+          const double Ax = apply_row(g, R, k0, u, fc, fm, fp, f0[u], f1[u], f2[u]);
+          ro[u] = 0.0;
+          if (R.in) {
+            const double vol = C.area * lv[k0 + u], res = bb[u] - avec * C.area * lv[k0 + u] - Ax;
+            ro[u] = res;
+            acc[0] += res * res;
+            acc[1] += fabs(res);
+            acc[2] += fc[u] * vol;
+          }
+        }
+        st4(r + s0, ro);
+      });
   write_partials<3>(acc, P.c);
 }
 
-__global__ __launch_bounds__(NSX_BLOCK) void k_modal_fold(Geo g, double *x, float *e, Partials P, SolverState *st,
-                                                           int cap) {
-  if (st->done) return;
-  const int iters = st->m_iters;
-  double t[3];
-  reduce_partials<3>(P.c, gridDim.x, t);
-  const double rN = sqrt(t[0]), e1 = t[1] / st->b1, e2 = rN / st->b2;
-  const bool finite = isfinite(t[0]) && isfinite(t[1]);
+// The reference's rules on the residual just formed: at the start (first)
+// the norms of b and r0 from k_resid and the no-solve test
+// (bicgstab.F90:453-469), later the stopping rule (:544-575).  Sets how far
+// the next cycle's 2D solves go: 1/200 of what is left to eps (at 1/20 the
+// pressure of a solve to 1e-13 was 3e-13 to 1e-12 from the 64-bit one, ten times
+// what it is now), no further than 1e-12.  Three cycles in a row that do not
+// lower the residual by a tenth, or the cap, end the solve (the FP64
+// BiCGSTAB goes on).
+__global__ __launch_bounds__(NSX_BLOCK) void k_modal_check(Geo g, Partials P, SolverState *st, int first, int cap) {
+  if (!first && st->done) return;
+  double e1, e2, xvol, rr;
   int stop = 0, code = EXIT_CONVERGED;
-  if (!finite) {
-    stop = 1;
-    code = EXIT_BREAKDOWN;
-  } else if (e1 < st->eps || e2 < st->eps) {
-    stop = 1;
-  } else if (iters >= cap) {
-    stop = 1;
-    code = EXIT_MAX;
+  const double last = st->m_e;
+  int stall = st->m_stall;
+  if (first) {
+    double t[5];
+    reduce_partials<5>(P.init, g.grid, t);
+    const double b2 = t[0] > 0.0 ? sqrt(t[0]) : 1.0, b1 = t[2] == 0.0 ? 1.0 : t[2];
+    rr = t[1];
+    e2 = sqrt(t[1]) / b2;
+    e1 = t[3] / b1;
+    xvol = t[4];
+    stall = 0;
+    if (threadIdx.x == 0) {
+      st->b1 = b1;
+      st->b2 = b2;
+    }
+    if (e1 < st->eps || e2 < st->eps) {
+      stop = 1;
+      code = EXIT_NO_SOLVE;
+    }
+  } else {
+    double t[3];
+    reduce_partials<3>(P.c, g.grid, t);
+    rr = t[0];
+    e2 = sqrt(t[0]) / st->b2;
+    e1 = t[1] / st->b1;
+    xvol = t[2];
+    if (e1 < st->eps || e2 < st->eps) stop = 1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  const double e = e1 < e2 ? e1 : e2;
+  if (!stop) {
+    if (!isfinite(rr) || !isfinite(e)) {
+      stop = 1;
+      code = EXIT_BREAKDOWN;
+    } else if (!first) {
+      stall = e > 0.9 * last ? stall + 1 : 0;
+      if (st->m_iters >= cap || stall == 3) {
+        stop = 1;
+        code = EXIT_MAX;
+      }
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
     st->e1 = e1;
     st->e2 = e2;
-    st->xvol = t[2];
-    st->a_iter = iters;
-    st->mp_pass += 1;
-    st->m_stop = 0;
+    st->xvol = xvol;
+    st->m_e = e;
+    st->m_stall = stall;
+    st->m_tau = fmax(0.005 * st->eps / e, 1e-12);
+    st->a_iter = st->m_iters;
     if (stop) {
       st->done = 1;
       st->exit_code = code;
     }
   }
-  // x += e, e = 0 (x keeps its value when the residual was not finite)
-  for_each_quad(g, [&](int, int k0, size_t s0) {
-    float ee[4];
-    ld4(e + s0, ee);
-    if (finite)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (k0 + v >= 1 && k0 + v <= g.NZ - 2) x[s0 + v] = x[s0 + v] + (double)ee[v];
-    const float z[4] = {0.f, 0.f, 0.f, 0.f};
-    st4(e + s0, z);
-  });
 }
 
-int launch_modal_spmv(const Geo &g, hipStream_t s, const ModalDev &M, const float *u, const float *pin, float *pout,
-                      float *w, Partials part, SolverState *st, int first, hipEvent_t *ev) {
-  LAUNCH_TIMED(ev, 0, k_modal_spmv, dim3(g.grid), dim3(NSX_BLOCK), cgs_lds(g), s, g, u, pin, pout, w, part, st,
-               first, (uint32_t)M.agrid);
+int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, const double *x, double *r, Partials part,
+                      const SolverState *st, hipEvent_t *ev) {
+  LAUNCH_TIMED(ev, 0, k_modal_true, dim3(g.grid), dim3(NSX_BLOCK), level_lds(g, sizeof(double)), s, g, rhs, x, r,
+               part, st);
   return (int)hipGetLastError();
 }
 
-int launch_modal_update(const Geo &g, hipStream_t s, const float *p, const float *w, float *e, float *r,
-                        Partials part, SolverState *st, hipEvent_t *ev) {
-  LAUNCH_TIMED(ev, 0, k_modal_update, dim3(g.grid), dim3(NSX_BLOCK), 0, s, g, p, w, e, r, part, st);
-  return (int)hipGetLastError();
-}
-
-int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, double *x, float *e, float *r, Partials part,
-                      SolverState *st, int cap) {
-  hipLaunchKernelGGL(k_modal_true, dim3(g.grid), dim3(NSX_BLOCK), 0, s, g, rhs, (const double *)x, (const float *)e,
-                     r, part, st);
-  hipLaunchKernelGGL(k_modal_fold, dim3(g.grid), dim3(NSX_BLOCK), 0, s, g, x, e, part, st, cap);
+int launch_modal_check(const Geo &g, hipStream_t s, Partials part, SolverState *st, int first, int cap) {
+  hipLaunchKernelGGL(k_modal_check, dim3(1), dim3(NSX_BLOCK), 0, s, g, part, st, first, cap);
   return (int)hipGetLastError();
 }

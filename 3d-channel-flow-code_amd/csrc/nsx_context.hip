@@ -112,12 +112,13 @@ struct nsx_ctx {
   int hslot[2] = {0, 0}, nhist[2] = {0, 0};
   double *pguess = nullptr;
   int guess_stage = -1;
-  // the vertical-mode preconditioner (NSX_REFINE_MODAL): the column graph
-  // kept from nsx_commit, the device tables once built
+  // the vertical-mode solve (NSX_REFINE_MODAL): the column graph kept from
+  // nsx_commit, the device tables once built, the cycles of the last solve
   std::vector<int> h_nbr;
   std::vector<double> h_ppec;
   ModalDev modal{};
   bool modal_ok = false;
+  int modal_cycles = 0;
   int iter_hint_cg = 0;
   int iter_hint_cgs = 0;
   int iter_hint_cgs64 = 0;
@@ -127,7 +128,7 @@ struct nsx_ctx {
   size_t evused = 0;
   Timer t_k[3], t_stage, t_cg[2];  // FP64 A, B, C; stage kernels; FP32 CG W, X
   Timer t_cgs, t_cgs64;              // single-reduction CG, FP32 and FP64
-  Timer t_mod[5];                    // vertical-mode CG: forward transform, V-cycle, backward, product, update
+  Timer t_mod[5];                    // vertical-mode solve: forward transform, 2D solves, backward, true residual
   // (event index, timer: 0..2 FP64 solver, 5 stage, 12..13 FP32 CG, 14 single-reduction CG, 15 its FP64 instance)
   std::vector<std::pair<size_t, int>> pending;
 };
@@ -1090,183 +1091,164 @@ static int solve_cgs(nsx_ctx *ctx, const double *rhs, const double *phi_in, doub
   return 0;
 }
 
-// the vertical-mode preconditioner's tables (nsx_modal.hip), built on the
-// host and uploaded at the first solve that uses them
+// the vertical-mode solve's tables (nsx_modal.hip), built on the host and
+// uploaded at the first solve that uses them
 static int modal_setup(nsx_ctx *ctx) {
   if (ctx->modal_ok) return 0;
-  const Geo &g = ctx->g;
   const int N0 = ctx->N0, NZ = ctx->NZ, nzi = NZ - 2;
-  // vertical couplings per unit area: between interior layers k and k+1,
-  // 1/dsig(k) (the quotient area/dsig(k) of the rows); a coupling to a ghost
-  // layer that is not Neumann stays on the diagonal
-  std::vector<double> tlay((size_t)nzi + 1, 0.0), svl((size_t)nzi);
-  for (int k = 1; k <= NZ - 3; ++k) tlay[k] = 1.0 / ctx->dsig[k];
-  tlay[0] = g.bcbot == 1 ? 0.0 : 1.0 / ctx->dsig[0];
-  tlay[nzi] = g.bctop == 1 ? 0.0 : 1.0 / ctx->dsig[NZ - 2];
+  // vertical couplings per unit area between interior layers k and k+1,
+  // 1/dsig(k) (the quotient area/dsig(k) of the rows)
+  std::vector<double> tlay((size_t)nzi, 0.0), svl((size_t)nzi);
+  for (int k = 1; k <= NZ - 3; ++k) tlay[k - 1] = 1.0 / ctx->dsig[k];
   for (int k = 1; k <= NZ - 2; ++k) svl[k - 1] = ctx->dsigv[k - 1];
   ModalHost H;
   std::string err;
-  const int m0 = std::min(NSX_MODAL_M0, nzi);
   if (modal_build_host(N0, nzi, ctx->h_nbr.data(), ctx->h_ppec.data(), ctx->areaCell.data(), tlay.data(),
-                       svl.data(), m0, H, err))
+                       svl.data(), H, err))
     return nsx_fail(ctx, -1, "%s", err.c_str());
+  hipDeviceProp_t prop;
+  HIPCHECK(hipGetDeviceProperties(&prop, ctx->dev));
+  const int lds = (int)std::max(prop.sharedMemPerBlockOptin, (size_t)65536);
   ModalDev &M = ctx->modal;
   M = ModalDev{};
-  const int nzp = (nzi + 3) / 4 * 4, MP = (nzi + 15) / 16 * 16, MT = MP / 16;
-  M.m0 = H.m0;
   M.nzi = nzi;
-  M.nzp = nzp;
-  M.mp = MP;
-  M.mt = MT;
+  M.N0 = N0;
+  M.N0p = (N0 + 15) / 16 * 16;
+  M.kt = (nzi + 15) / 16;
   M.nlev = (int)H.levels.size();
   M.nc = H.nc;
+  // the transforms' panels: the most output tiles whose part of the table
+  // fits the LDS (and the accumulators eight), spread evenly
+  const int tile = M.kt * 256 * (int)sizeof(double), most = std::min(8, lds / tile);
+  if (most < 1) return nsx_fail(ctx, -1, "vertical-mode solve: %d layers pass the mode table's LDS", nzi);
+  M.npanel = (M.kt + most - 1) / most;
+  M.mt = (M.kt + M.npanel - 1) / M.npanel;
   {
-    // transform blocks: two per CU, four waves of 16 columns each (the
-    // vector-unit transforms take the same grid)
-    hipDeviceProp_t prop;
-    HIPCHECK(hipGetDeviceProperties(&prop, ctx->dev));
-    const int waves = (N0 + 15) / 16, want = (waves + 3) / 4;
-    M.agrid = std::max(1, std::min(want, 2 * prop.multiProcessorCount));
-    M.lds_optin = (int)std::max(prop.sharedMemPerBlockOptin, (size_t)65536);
+    // as many blocks as are resident, four waves of 16 columns each
+    const int per = std::max(1, std::min(4, lds / (M.mt * tile))), want = (M.N0p / 16 + 3) / 4;
+    M.agrid = std::max(1, std::min(want, std::max(1, per * prop.multiProcessorCount / M.npanel)));
   }
-  std::vector<float> ph((size_t)nzp * nzp, 0.f), pt((size_t)nzp * nzp, 0.f), mu((size_t)MP, 1.f);
-  for (int k = 0; k < nzi; ++k)
-    for (int m = 0; m < nzi; ++m) {
-      ph[(size_t)k * nzp + m] = H.phi[(size_t)k * nzi + m];
-      pt[(size_t)m * nzp + k] = H.phi[(size_t)k * nzi + m];
-    }
-  for (int m = 0; m < nzi; ++m) mu[m] = H.mu[m];
-  // matrix-core operands: forward, lane (j, q4) of (layer group t, mode tile
-  // mt) holds phi(16 t + 4 q4 + q, 16 mt + j); backward, of (mode group t,
-  // layer tile nt), phi(16 nt + j, 16 t + 4 q4 + q)
-  auto phik = [&](int k, int m) -> float { return (k < nzi && m < nzi) ? H.phi[(size_t)k * nzi + m] : 0.f; };
-  std::vector<float> tf((size_t)MT * MT * 256, 0.f), tb((size_t)MT * MT * 256, 0.f);
-  for (int t = 0; t < MT; ++t)
-    for (int mt = 0; mt < MT; ++mt)
+  const int MP = 16 * M.kt, ntab = M.npanel * M.mt * M.kt * 256;
+  auto phik = [&](int k, int m) -> double { return (k < nzi && m < nzi) ? H.phi[(size_t)k * nzi + m] : 0.0; };
+  std::vector<double> tf((size_t)ntab, 0.0), tb((size_t)ntab, 0.0), mu((size_t)MP, 1.0);
+  for (int o = 0; o < M.npanel * M.mt; ++o)
+    for (int t = 0; t < M.kt; ++t)
       for (int lane = 0; lane < 64; ++lane)
         for (int q = 0; q < 4; ++q) {
-          const int j = lane & 15, q4 = lane >> 4;
-          tf[(((size_t)t * MT + mt) * 64 + lane) * 4 + q] = phik(16 * t + 4 * q4 + q, 16 * mt + j);
-          tb[(((size_t)t * MT + mt) * 64 + lane) * 4 + q] = phik(16 * mt + j, 16 * t + 4 * q4 + q);
+          const int out = 16 * o + (lane & 15), in = 16 * t + 4 * (lane >> 4) + q;
+          const size_t at = (((size_t)o * M.kt + t) * 64 + lane) * 4 + q;
+          tf[at] = phik(in, out);
+          tb[at] = phik(out, in);
         }
-  int rc;
-  float *d_ph, *d_pt, *d_mu, *d_ci, *d_xh, *d_tf, *d_tb;
-  if ((rc = dev_upload(ctx, &d_ph, ph)) || (rc = dev_upload(ctx, &d_pt, pt)) || (rc = dev_upload(ctx, &d_mu, mu)) ||
-      (rc = dev_upload(ctx, &d_tf, tf)) || (rc = dev_upload(ctx, &d_tb, tb)) ||
-      (rc = dev_alloc(ctx, &d_xh, (size_t)N0 * MP)))
-    return rc;
-  {
-    // the coarsest inverses laid out [J][K][m] for coalesced reads
-    const int nc = H.nc, m0v = H.m0;
-    std::vector<float> ct((size_t)nc * nc * m0v, 0.f);
-    for (int m = 0; m < m0v; ++m)
-      for (int J = 0; J < nc; ++J)
-        for (int K = 0; K < nc; ++K)
-          ct[((size_t)J * nc + K) * m0v + m] = H.cinv[((size_t)m * nc + J) * nc + K];
-    if ((rc = dev_upload(ctx, &d_ci, ct))) return rc;
+  std::copy(H.mu.begin(), H.mu.end(), mu.begin());
+  std::vector<float> wa((size_t)N0 * 4);
+  for (int i = 0; i < N0; ++i) {
+    for (int j = 0; j < 3; ++j) wa[(size_t)i * 4 + j] = (float)H.w[(size_t)i * 3 + j];
+    wa[(size_t)i * 4 + 3] = (float)ctx->areaCell[i];
   }
-  HIPCHECK(hipMemset(d_xh, 0, (size_t)N0 * MP * sizeof(float)));
-  M.phi = d_ph;
-  M.phiT = d_pt;
-  M.tfwd = reinterpret_cast<const float4 *>(d_tf);
-  M.tbwd = reinterpret_cast<const float4 *>(d_tb);
-  M.mu = d_mu;
-  M.cinv = d_ci;
-  M.xh = d_xh;
+  int rc;
+  auto up = [&](const auto &v, auto *&dst) -> int {
+    std::remove_const_t<std::remove_reference_t<decltype(*dst)>> *q;
+    const int r = dev_upload(ctx, &q, v);
+    dst = q;
+    return r;
+  };
+  const float *d_wa;
+  if ((rc = up(tf, M.tfwd)) || (rc = up(tb, M.tbwd)) || (rc = up(mu, M.mu)) || (rc = up(H.cinv, M.cinv)) ||
+      (rc = up(H.nb, M.nb)) || (rc = up(wa, d_wa)) || (rc = up(H.w, M.w64)) ||
+      (rc = up(std::vector<double>(ctx->areaCell.begin(), ctx->areaCell.begin() + N0), M.area64)))
+    return rc;
+  M.wa = reinterpret_cast<const float4 *>(d_wa);
   for (int l = 0; l < M.nlev; ++l) {
     const ModalHost::Level &h = H.levels[l];
     ModalLevelDev &d = M.lev[l];
     d.n = h.n;
-    auto up_i = [&](const std::vector<int> &v, const int *&dst) -> int {
-      if (v.empty()) return 0;
-      int *q;
-      const int r = dev_upload(ctx, &q, v);
-      dst = q;
-      return r;
-    };
-    auto up_f = [&](const std::vector<float> &v, const float *&dst) -> int {
-      if (v.empty()) return 0;
-      float *q;
-      const int r = dev_upload(ctx, &q, v);
-      dst = q;
-      return r;
-    };
-    if ((rc = up_i(h.ptr, d.ptr)) || (rc = up_i(h.col, d.col)) || (rc = up_f(h.w, d.w)) ||
-        (rc = up_f(h.diag, d.diag)) || (rc = up_f(h.area, d.area)) || (rc = up_i(h.agg, d.agg)) ||
-        (rc = up_i(h.eagg, d.eagg)) || (rc = up_i(h.dptr, d.dptr)) || (rc = up_i(h.dcol, d.dcol)) ||
-        (rc = up_f(h.db, d.db)) || (rc = up_f(h.dz, d.dz)))
-      return rc;
-    const size_t nm = (size_t)h.n * (size_t)M.m0;
-    if ((rc = dev_alloc(ctx, &M.b[l], nm)) || (rc = dev_alloc(ctx, &M.z[l], nm)) ||
-        (rc = dev_alloc(ctx, &M.x[l], nm)))
-      return rc;
-    HIPCHECK(hipMemset(M.x[l], 0, nm * sizeof(float)));
+    if ((rc = up(h.diag, d.diag)) || (rc = up(h.area, d.area)) || (rc = up(h.sabs, d.sabs))) return rc;
+    const SellHost *hs[3] = {&h.A, &h.R, &h.P};
+    SellDev *ds[3] = {&d.A, &d.R, &d.P};
+    for (int q = 0; q < 3; ++q)
+      if (hs[q]->n && ((rc = up(hs[q]->ptr, ds[q]->ptr)) || (rc = up(hs[q]->col, ds[q]->col)) ||
+                       (rc = up(hs[q]->val, ds[q]->val))))
+        return rc;
   }
+  // the 2D blocks' vectors: into LDS from the coarsest level up while they
+  // fit (gathered vectors first), the others into the mode's workspace
+  int used = 0, work = 0;
+  const int cap = (lds - 2048) / (int)sizeof(float);
+  auto place = [&](VecLoc &v, int n) {
+    n = (n + 15) / 16 * 16;
+    v.lds = used + n <= cap;
+    int &at = v.lds ? used : work;
+    v.off = at;
+    at += n;
+  };
+  for (int l = M.nlev - 1; l >= 1; --l) {
+    place(M.lev[l].y, M.lev[l].n);
+    place(M.lev[l].t, M.lev[l].n);
+    place(M.lev[l].b, M.lev[l].n);
+  }
+  place(M.lev[0].y, N0);
+  place(M.z0, N0);
+  place(M.p[0], N0);
+  place(M.p[1], N0);
+  M.lds2d = used * (int)sizeof(float);
+  M.nwork = work;
+  if (!modal_allow_lds(M)) return nsx_fail(ctx, -2, "vertical-mode solve: the kernels' LDS limit cannot be raised");
+  const size_t nm = (size_t)MP * M.N0p;
+  if ((rc = dev_alloc(ctx, &M.bh, nm)) || (rc = dev_alloc(ctx, &M.xh, nm)) || (rc = dev_alloc(ctx, &M.ap, nm)) ||
+      (rc = dev_alloc(ctx, &M.work, (size_t)nzi * work)) ||
+      (rc = dev_alloc(ctx, &M.part, (size_t)M.agrid * M.npanel)))
+    return rc;
+  HIPCHECK(hipMemsetAsync(M.xh, 0, nm * sizeof(double), ctx->stream));
   ctx->modal_ok = true;
   return 0;
 }
 
-// Mixed precision, NSX_REFINE_MODAL: FP32 CG preconditioned by the vertical
-// modes (launch_modal_apply) in cycles.  e gathers a cycle's correction in
-// FP32; a cycle starts from the true FP64 residual with beta = 0 and ends
-// when rho has fallen by NSX_MODAL_DROP (FP32 recursion holds the residual to
-// about 1e-5 of the cycle's start; keeping p across the update, the next beta
-// would divide the true residual's rho by the drifted recursive one) or after
-// the iterations launched for it.  Then the true FP64 residual of x + e
-// replaces r, e joins x and the reference's stopping rule is tested on it.
-// The cap and a breakdown leave x at its last update and the FP64 BiCGSTAB
-// finishes, as for the other CG forms.
+// Mixed precision, NSX_REFINE_MODAL: cycles of the vertical-mode solve, each
+// from the true FP64 residual: transform it, solve every mode's 2D problem
+// (FP64 CG with an FP32 multigrid preconditioner), transform back into x.
+// The reference's stopping rule is tested on the true residual after each
+// cycle.  The cap, a breakdown and a residual that stops falling leave x at
+// its last update and the FP64 BiCGSTAB finishes, as for the CG forms.
 static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, double *x) {
   int rc = modal_setup(ctx);
   if (rc) return rc;
   const Geo &g = ctx->g;
   hipStream_t s = ctx->stream;
   const int cap = 2 * ctx->MaxIters + 100;
-  // r0 = b - A x0 (FP32 into frhat), e = 0, x = x0, the norms of b and the
-  // reference's no-solve test
-  LAUNCH(launch_cg_init(g, s, rhs, phi_in, x, ctx->fr, ctx->frhat, ctx->fe, ctx->part, ctx->st_dev, ctx->eps,
-                        ctx->delta_cg, cap));
-  float *r = ctx->frhat, *u = ctx->fr, *w = ctx->fv, *e = ctx->fe;
-  float *p[2] = {ctx->fp, ctx->fp2};
-  HIPCHECK(hipMemcpyAsync(ctx->st_host, ctx->st_dev, sizeof(SolverState), hipMemcpyDeviceToHost, s));
-  HIPCHECK(hipStreamSynchronize(s));
-  int launched = 0, cycle = NSX_MODAL_FIRST, before = 0;
-  if (!ctx->st_host->done) {
-    for (;;) {
-      const size_t pend0 = ctx->pending.size();
-      for (int c = 0; c < cycle; ++c) {
-        // with timing: start/stop pairs of the forward transform, the
-        // V-cycle, the backward transform, the product and the update
-        hipEvent_t *ev = nullptr;
-        if (ctx->timing) {
-          ev = events(ctx, 10);
-          if (!ev) return nsx_fail(ctx, -2, "hipEventCreate failed");
-        }
-        LAUNCH(launch_modal_apply(g, s, ctx->modal, r, u, ctx->part, ctx->st_dev, ev));
-        LAUNCH(launch_modal_spmv(g, s, ctx->modal, u, p[launched & 1], p[(launched + 1) & 1], w, ctx->part,
-                                 ctx->st_dev, c == 0, ev ? ev + 6 : nullptr));
-        LAUNCH(launch_modal_update(g, s, p[(launched + 1) & 1], w, e, r, ctx->part, ctx->st_dev,
-                                   ev ? ev + 8 : nullptr));
-        if (ev) {
-          const size_t base = (size_t)(ev - &ctx->evpool[0]);
-          for (int q = 0; q < 5; ++q) ctx->pending.push_back({base + 2 * q, 16 + q});
-        }
-        ++launched;
+  double *r = ctx->srhat;
+  // x = x0, r = b - A x0, the norms of b and the no-solve test
+  LAUNCH(launch_bicg_init(g, s, rhs, phi_in, x, ctx->sr, r, ctx->part, ctx->st_dev, ctx->eps, ctx->MaxIters));
+  LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 1, cap));
+  const size_t pend0 = ctx->pending.size();
+  // as many cycles as the last solve took, then one at a time
+  for (int cycles = std::max(1, ctx->modal_cycles), issued = 0;; cycles = 1) {
+    for (int c = 0; c < cycles; ++c, ++issued) {
+      hipEvent_t *ev = nullptr;
+      if (ctx->timing) {
+        ev = events(ctx, 8);
+        if (!ev) return nsx_fail(ctx, -2, "hipEventCreate failed");
       }
-      LAUNCH(launch_modal_true(g, s, rhs, x, e, r, ctx->part, ctx->st_dev, cap));
-      HIPCHECK(hipMemcpyAsync(ctx->st_host, ctx->st_dev, sizeof(SolverState), hipMemcpyDeviceToHost, s));
-      HIPCHECK(hipStreamSynchronize(s));
-      const int used = ctx->st_host->m_iters - before;
-      before = ctx->st_host->m_iters;
-      // timing: only the iterations that ran (after a drop the launches return at once)
-      if (ctx->timing && ctx->pending.size() > pend0 + 5 * (size_t)used) ctx->pending.resize(pend0 + 5 * (size_t)used);
-      if (ctx->st_host->done) break;
-      // the next cycle: as long as this one ran, a few more
-      cycle = std::min(NSX_MODAL_CYCLE, std::max(8, used + 4));
+      LAUNCH(launch_modal_fwd(g, s, ctx->modal, r, ctx->st_dev, ev));
+      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, ev ? ev + 2 : nullptr));
+      LAUNCH(launch_modal_bwd(g, s, ctx->modal, x, ctx->st_dev, ev ? ev + 4 : nullptr));
+      LAUNCH(launch_modal_true(g, s, rhs, x, r, ctx->part, ctx->st_dev, ev ? ev + 6 : nullptr));
+      LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 0, cap));
+      if (ev) {
+        const size_t base = (size_t)(ev - &ctx->evpool[0]);
+        for (int q = 0; q < 4; ++q) ctx->pending.push_back({base + 2 * q, 16 + q});
+      }
     }
+    HIPCHECK(hipMemcpyAsync(ctx->st_host, ctx->st_dev, sizeof(SolverState), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipStreamSynchronize(s));
+    if (ctx->st_host->done) break;
+    if (issued > cap) return nsx_fail(ctx, -4, "solver did not stop after %d cycles", issued);
   }
-  collect_timing(ctx);
   const SolverState &h = *ctx->st_host;
+  // timing: the cycles that ran
+  if (ctx->timing && ctx->pending.size() > pend0 + 4 * (size_t)h.mp_pass) ctx->pending.resize(pend0 + 4 * (size_t)h.mp_pass);
+  collect_timing(ctx);
+  if (h.mp_pass > 0) ctx->modal_cycles = h.mp_pass;
   const int it = h.m_iters;
   if (h.exit_code == NSX_SOLVE_MAX_ITERS || h.exit_code == NSX_SOLVE_BREAKDOWN)
     return finish_fp64(ctx, rhs, x, it, h.mp_pass);

@@ -1,8 +1,20 @@
 // nsx_kernels.h -- launchers of the stage kernels (nsx_stage.hip) and of the
 // pressure solver (nsx_bicgstab.hip), called by the context (nsx_context.hip).
 #pragma once
+#include <hip/hip_ext.h>
+
 #include "nsx_dev.h"
 #include "nsx_modal.h"
+
+// With timing on, a kernel is launched with its own start/stop events
+// (recorded by the dispatch itself, so the elapsed time is the kernel's)
+#define LAUNCH_TIMED(ev, q, kern, grid, blk, lds, s, ...)                                         \
+  do {                                                                                          \
+    if (ev)                                                                                     \
+      hipExtLaunchKernelGGL(kern, grid, blk, lds, s, (ev)[2 * (q)], (ev)[2 * (q) + 1], 0, __VA_ARGS__); \
+    else                                                                                        \
+      hipLaunchKernelGGL(kern, grid, blk, lds, s, __VA_ARGS__);                                 \
+  } while (0)
 
 // Per-block partial sums of one reduction site: [rows][grid]
 struct Partials {
@@ -58,12 +70,13 @@ struct SolverState {
   CgsCarry cgs[2];   // single-reduction FP32 CG, by parity of the launch
   int cgs_runs;      // launches of the single-reduction CG that ran (block 0 of each)
   int pad3;
-  // the CG with the vertical-mode preconditioner (NSX_REFINE_MODAL)
-  double m_rho;       // rho_i = <r_i, M^-1 r_i> of the iteration running     (product kernel)
-  double m_rho_prev;  // rho of the last completed iteration                   (update kernel)
-  double m_rho0;      // rho of the cycle's first iteration                    (product kernel)
-  int m_stop;         // the cycle has met its drop: its remaining launches return (product kernel; fold: 0)
-  int m_iters;        // iterations completed                                   (update kernel)
+  // the vertical-mode solve (NSX_REFINE_MODAL)
+  double m_e;         // min(e1, e2) of the last residual                        (check kernel)
+  double m_tau;       // how far the next 2D solves go                           (check kernel)
+  int m_stall;        // cycles in a row that did not lower it by a tenth        (check kernel)
+  int m_cyc;          // most iterations of a mode in this cycle                 (2D solves; backward transform: 0)
+  int m_iters;        // sum of m_cyc over the cycles                            (backward transform)
+  int pad4;
 };
 
 // the vectors of the single-reduction CG: e and p in place, the scaled
@@ -193,26 +206,13 @@ int launch_cgs64(const Geo &g, hipStream_t s, int j, const double *rhs, double *
 int launch_gnorm_apply(const Geo &g, hipStream_t s, double *x, const SolverState *st);
 int launch_gnorm_sum(const Geo &g, hipStream_t s, const double *x, Partials part);
 
-// ---- the CG with the vertical-mode preconditioner (NSX_REFINE_MODAL)
-// u = M^-1 r (modal transform, the low modes' V-cycle, the others' diagonal,
-// transform back; u is stored at every slot, zero outside the interior) and
-// the partial sums of <r, u> into P.a
-// (ev: null, or six events: the forward transform's start and stop (recorded
-// by its dispatch), the V-cycle's start and stop (recorded on the stream
-// around its launches), the backward transform's start and stop)
-int launch_modal_apply(const Geo &g, hipStream_t s, const ModalDev &M, const float *r, float *u, Partials part,
-                       const SolverState *st, hipEvent_t *ev = nullptr);
-// p_out = u + beta p_in (beta = 0 when first: the cycle's first iteration) at
-// the seven points, w = A p_out, partials of <p, w> into P.b; rho from P.a
-// (M.agrid partials) kept in the state; a rho below NSX_MODAL_DROP times the
-// cycle's first ends the cycle (st->m_stop)
-int launch_modal_spmv(const Geo &g, hipStream_t s, const ModalDev &M, const float *u, const float *pin, float *pout,
-                      float *w, Partials part, SolverState *st, int first, hipEvent_t *ev = nullptr);
-// alpha = rho / <p, w>; e += alpha p, r -= alpha w
-int launch_modal_update(const Geo &g, hipStream_t s, const float *p, const float *w, float *e, float *r,
-                        Partials part, SolverState *st, hipEvent_t *ev = nullptr);
-// the true FP64 residual of x + e into r and its partials (P.c); then x += e,
-// e = 0, a new cycle (m_stop = 0) and the reference's stopping rule (st: e1,
-// e2, xvol, done, exit code; the iteration cap after st->m_iters iterations)
-int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, double *x, float *e, float *r, Partials part,
-                      SolverState *st, int cap);
+// ---- the vertical-mode solve (NSX_REFINE_MODAL): x -= Phi (2D solves of
+// Phi^T r), r = b - A x, the stopping rule.  ev: null, or the dispatch's start and stop
+int launch_modal_fwd(const Geo &g, hipStream_t s, const ModalDev &M, const double *r, SolverState *st,
+                     hipEvent_t *ev);
+int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, hipEvent_t *ev);
+int launch_modal_bwd(const Geo &g, hipStream_t s, const ModalDev &M, double *x, SolverState *st, hipEvent_t *ev);
+int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, const double *x, double *r, Partials part,
+                      const SolverState *st, hipEvent_t *ev);
+int launch_modal_check(const Geo &g, hipStream_t s, Partials part, SolverState *st, int first, int cap);
+bool modal_allow_lds(const ModalDev &M);

@@ -140,34 +140,18 @@ CGS_KERNEL = {4: "k_cgs<float, 0>", 5: "k_cgs<float, 1>", 6: "k_cgs<float, 2>"}
 
 def modal_kernels(case) -> dict:
     """timer -> (kernel name, algorithmic bytes per launch) of the vertical-mode
-    CG: the forward transform reads r and writes the modal coefficients (and
-    z = b / d of the 16 multigrid modes); the backward one reads them (and b
-    and z of the multigrid modes where it forms the level-0 post-smoothing)
-    and r and writes u; the product reads u and p and writes p and w; the update
-    reads p, w, e, r and writes e and r (FP32, interior prisms)"""
-    n0, nzi = case.N_CELL0, case.NZ - 2
-    mt = (nzi + 15) // 16
-    m0 = min(16, nzi)
-    n = case.n_interior
-    # the staged transforms where table and staging fit the LDS a block may
-    # opt into (the MI355X allowed the 98 KB of the 128-layer workload; 160 KB
-    # is the CU's LDS)
-    lds_optin = 160 * 1024
-    fstaged = mt * mt * 1024 + 4 * 16 * 16 * mt * 4 <= lds_optin
-    fwd = ("k_modal_fwd_mfma<%d, %s>" % (mt, "true" if fstaged else "false")) if mt <= 8 else "k_modal_fwd_vec"
-    ns = (case.NZ + 3) // 4 * 4
-    staged = mt * mt * 1024 + 4 * 16 * ns * 4 <= lds_optin
-    # the backward transform forms the level-0 post-smoothing where there are
-    # 16 multigrid modes and more than one level (over 400 columns)
-    v0 = mt <= 8 and nzi >= 16 and n0 > 400
-    bwd = ("k_modal_bwd_mfma<%d, %s, %s>" % (mt, "true" if staged else "false", "true" if v0 else "false")
-           if mt <= 8 else "k_modal_bwd_vec")
-    # (the backward transform with the level-0 post-smoothing also reads b
-    # and z of the 16 multigrid modes: the level below's x is counted as
-    # cached)
-    return {"modal_fwd": (fwd, 4 * (2 * n + n0 * m0)), "modal_bwd": (bwd, 4 * (3 * n + (2 * n0 * m0 if v0 else 0))),
-            "modal_spmv": ("k_modal_spmv", 16 * n), "modal_update": ("k_modal_update", 24 * n),
-            "modal_mg": ("V-cycle (k_mg_down, k_mg_coarse, k_mg_up)", 0)}
+    solve: the forward transform reads r and writes the modal right-hand
+    sides; the backward one reads the modal solutions and reads and writes x;
+    the true residual reads b and x and writes r (FP64, interior prisms).  The
+    2D solves' time is that of a whole cycle (their iterations vary by mode)"""
+    n, nzi = case.n_interior, case.NZ - 2
+    kt = (nzi + 15) // 16
+    # output tiles a block forms: what of the table fits 160 KB of LDS, at most 8
+    most = max(1, min(8, 160 * 1024 // (kt * 2048)))
+    panels = (kt + most - 1) // most
+    mt = (kt + panels - 1) // panels
+    return {"modal_fwd": ("k_modal_fwd<%d>" % mt, 16 * n), "modal_bwd": ("k_modal_bwd<%d>" % mt, 24 * n),
+            "modal_spmv": ("k_modal_true", 24 * n), "modal_mg": ("2D solves of every mode", 0)}
 
 
 def leg(case, name: str, steps: int, warmup: int, eps: float, max_iters=None, guess: int = 0) -> dict:

@@ -1,0 +1,80 @@
+"""The vertical-mode solve (NSX_REFINE_MODAL) at the sizes where its parts end:
+meshes of one, two and more levels of the 2D hierarchy, layers either side of
+a 16-wide tile of the transforms, columns either side of a 16-column tile,
+tables that need several panels, vectors that pass the LDS of a block, walls.
+A random right-hand side solved to eps: the host-checked residual meets the
+reference's rule (2 eps for the summation order), and the pressure agrees
+with the FP64 BiCGSTAB's to what the two stopping errors allow (eps times the
+operator's condition number, below 1e4 here: 1e-6)."""
+import numpy as np
+import pytest
+
+from common import bc_case, interior, load_bc, ppe_residual, rel_err
+from nsx.abi import PREC_MIXED, REFINE_MODAL
+from nsx.case import make_case
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-10
+
+
+def _check(c, seed):
+    from nsx.device import Context
+    rng = np.random.default_rng(seed)
+    rhs = c.cell_field()
+    rhs[:c.N_CELL0, 1:-1] = rng.standard_normal((c.N_CELL0, c.NZ - 2))
+    G = Context(c)
+    G.set_params(eps=EPS)
+    G.init_state()
+    phi64, pv64, _ = G.bicgstab(c.cell_field(), rhs)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    phi, pv, info = G.bicgstab(c.cell_field(), rhs)
+    again, _, _ = G.bicgstab(c.cell_field(), rhs)
+    G.close()
+    assert info["exit"] == "converged" and info["iters_fp32"] > 0, info
+    e1, e2 = ppe_residual(c, phi, rhs)
+    assert min(e1, e2) < 2 * EPS, (e1, e2)
+    assert rel_err(interior(c, phi), interior(c, phi64)) <= 1e-6
+    assert rel_err(pv, pv64) <= 1e-6
+    assert np.array_equal(phi, again), "two runs of the same solve differ"
+
+
+@pytest.mark.parametrize("nx, ny, nn", [
+    (2, 2, 2),       # 8 columns, one level, two layers
+    (8, 6, 15),      # 96 columns: the largest single level; one layer short of a tile
+    (7, 7, 16),      # 98 columns: two levels, a column tile of two
+    (13, 9, 17),     # one layer past a tile, odd columns
+    (40, 21, 33),    # 1,680 columns, three levels
+    (12, 8, 130),    # two panels
+    (12, 8, 260),    # seventeen tiles, one past the eight a block accumulates twice over
+    (90, 41, 9),     # 7,380 columns: the columns' vectors pass the block's LDS
+])
+def test_modal_sizes(nx, ny, nn):
+    _check(make_case(nx, ny, nn, seed=11, jitter=0.1), seed=nx + nn)
+
+
+@pytest.mark.parametrize("walls", [(1, 0, 0, 0), (0, 0, 0, 0), (0, 1, 1, 1)])
+def test_modal_walls_odd(walls):
+    _check(make_case(27, 15, 19, seed=5, jitter=0.1, walls=walls), seed=3)
+
+
+def test_modal_zero_and_solved_right_hand_sides():
+    """A zero right-hand side and one solved already take no iterations; the pressure
+    stays."""
+    from nsx.device import Context
+    c = bc_case(load_bc(), "duct", "steps")
+    G = Context(c)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    G.init_state()
+    zero = c.cell_field()
+    phi, _, info = G.bicgstab(zero, zero)
+    assert info["exit"] == "no solve" and info["iters"] == 0, info
+    assert not np.any(interior(c, phi))
+    rhs = c.cell_field()
+    rhs[:c.N_CELL0, 1:-1] = np.random.default_rng(2).standard_normal((c.N_CELL0, c.NZ - 2))
+    phi, _, info = G.bicgstab(zero, rhs)
+    assert info["exit"] == "converged"
+    again, _, info = G.bicgstab(phi, rhs)
+    G.close()
+    assert info["exit"] == "no solve" and info["iters"] == 0, info
+    assert rel_err(interior(c, again), interior(c, phi)) <= 1e-12
