@@ -118,7 +118,7 @@ struct nsx_ctx {
   std::vector<double> h_ppec;
   ModalDev modal{};
   bool modal_ok = false;
-  int modal_cycles = 0;
+  int modal_cycles = 0, modal_iters = 44;
   int iter_hint_cg = 0;
   int iter_hint_cgs = 0;
   int iter_hint_cgs64 = 0;
@@ -1117,6 +1117,8 @@ static int modal_setup(nsx_ctx *ctx) {
   M.kt = (nzi + 15) / 16;
   M.nlev = (int)H.levels.size();
   M.nc = H.nc;
+  M.mp = 16 * M.kt;
+  M.batched = N0 >= NSX_MODAL_BATCH && M.nlev >= 3 && M.mp <= 4 * NSX_BLOCK;
   // the transforms' panels: the most output tiles whose part of the table
   // fits the LDS (and the accumulators eight), spread evenly
   const int tile = M.kt * 256 * (int)sizeof(double), most = std::min(8, lds / tile);
@@ -1163,13 +1165,39 @@ static int modal_setup(nsx_ctx *ctx) {
     const ModalHost::Level &h = H.levels[l];
     ModalLevelDev &d = M.lev[l];
     d.n = h.n;
-    if ((rc = up(h.diag, d.diag)) || (rc = up(h.area, d.area)) || (rc = up(h.sabs, d.sabs))) return rc;
+    if ((rc = up(h.diag, d.diag)) || (rc = up(h.area, d.area))) return rc;
+    const bool rows = M.batched && l <= 1;  // these levels' matrices row by row, the others' in slices
     const SellHost *hs[3] = {&h.A, &h.R, &h.P};
     SellDev *ds[3] = {&d.A, &d.R, &d.P};
+    const CsrHost *hc[3] = {&h.Ac, &h.Rc, &h.Pc};
+    CsrDev *dc[3] = {&d.Ac, &d.Rc, &d.Pc};
     for (int q = 0; q < 3; ++q)
-      if (hs[q]->n && ((rc = up(hs[q]->ptr, ds[q]->ptr)) || (rc = up(hs[q]->col, ds[q]->col)) ||
-                       (rc = up(hs[q]->val, ds[q]->val))))
+      if (rows) {
+        if (hc[q]->n && ((rc = up(hc[q]->ptr, dc[q]->ptr)) || (rc = up(hc[q]->col, dc[q]->col)) ||
+                         (rc = up(hc[q]->val, dc[q]->val))))
+          return rc;
+      } else if (hs[q]->n && ((rc = up(hs[q]->ptr, ds[q]->ptr)) || (rc = up(hs[q]->col, ds[q]->col)) ||
+                              (rc = up(hs[q]->val, ds[q]->val)))) {
         return rc;
+      }
+    if ((l >= 1 || M.batched) && l + 1 < M.nlev) {
+      // Chebyshev on [max(lmax/4, lmin), lmax] per mode: Gershgorin's bound of
+      // D^-1 A above, mu area / diagonal below (L is semi-definite)
+      std::vector<Cheb> ch((size_t)MP);
+      for (int m = 0; m < MP; ++m) {
+        float lmax = 1.f, lmin = 1.f;
+        for (int i = 0; i < h.n; ++i) {
+          const float ma = (float)mu[m] * h.area[i], di = h.diag[i] + ma;
+          if (!(di > 0.f)) continue;
+          lmax = std::max(lmax, 1.f + h.sabs[i] / di);
+          lmin = std::min(lmin, ma / di);
+        }
+        const float lo = std::min(std::max(0.25f * lmax, lmin), 0.9f * lmax);
+        const float th = 0.5f * (lmax + lo), de = 0.5f * (lmax - lo), rho0 = de / th, rho1 = 1.f / (2.f * th / de - rho0);
+        ch[m] = {1.f / th, rho1 * rho0, 2.f * rho1 / de};
+      }
+      if ((rc = up(ch, d.cheb))) return rc;
+    }
   }
   // the 2D blocks' vectors: into LDS from the coarsest level up while they
   // fit (gathered vectors first), the others into the mode's workspace
@@ -1182,15 +1210,17 @@ static int modal_setup(nsx_ctx *ctx) {
     v.off = at;
     at += n;
   };
-  for (int l = M.nlev - 1; l >= 1; --l) {
+  for (int l = M.nlev - 1; l >= (M.batched ? 2 : 1); --l) {
     place(M.lev[l].y, M.lev[l].n);
     place(M.lev[l].t, M.lev[l].n);
     place(M.lev[l].b, M.lev[l].n);
   }
-  place(M.lev[0].y, N0);
-  place(M.z0, N0);
-  place(M.p[0], N0);
-  place(M.p[1], N0);
+  if (!M.batched) {
+    place(M.lev[0].y, N0);
+    place(M.z0, N0);
+    place(M.p[0], N0);
+    place(M.p[1], N0);
+  }
   M.lds2d = used * (int)sizeof(float);
   M.nwork = work;
   if (!modal_allow_lds(M)) return nsx_fail(ctx, -2, "vertical-mode solve: the kernels' LDS limit cannot be raised");
@@ -1200,6 +1230,19 @@ static int modal_setup(nsx_ctx *ctx) {
       (rc = dev_alloc(ctx, &M.part, (size_t)M.agrid * M.npanel)))
     return rc;
   HIPCHECK(hipMemsetAsync(M.xh, 0, nm * sizeof(double), ctx->stream));
+  if (M.batched) {
+    const size_t n0 = (size_t)N0 * MP, n1 = (size_t)M.lev[1].n * MP, n2 = (size_t)M.lev[2].n * MP;
+    float **v[11] = {&M.R, &M.V, &M.Z, &M.W, &M.P[0], &M.P[1], &M.y1, &M.t1, &M.b1, &M.y2, &M.b2};
+    for (int q = 0; q < 11; ++q) {
+      const size_t n = q < 6 ? n0 : q < 9 ? n1 : n2;
+      if ((rc = dev_alloc(ctx, v[q], n))) return rc;
+      HIPCHECK(hipMemsetAsync(*v[q], 0, n * sizeof(float), ctx->stream));
+    }
+    if ((rc = dev_alloc(ctx, &M.ms, MP)) || (rc = dev_alloc(ctx, &M.rpart, NSX_MB_MEAN)) ||
+        (rc = dev_alloc(ctx, &M.rpart2, (size_t)NSX_MB_GRID * MP)) ||
+        (rc = dev_alloc(ctx, &M.nact, NSX_MB_ITERS + 1)))
+      return rc;
+  }
   ctx->modal_ok = true;
   return 0;
 }
@@ -1230,7 +1273,7 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
         if (!ev) return nsx_fail(ctx, -2, "hipEventCreate failed");
       }
       LAUNCH(launch_modal_fwd(g, s, ctx->modal, r, ctx->st_dev, ev));
-      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, ev ? ev + 2 : nullptr));
+      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, ctx->modal_iters, ev ? ev + 2 : nullptr));
       LAUNCH(launch_modal_bwd(g, s, ctx->modal, x, ctx->st_dev, ev ? ev + 4 : nullptr));
       LAUNCH(launch_modal_true(g, s, rhs, x, r, ctx->part, ctx->st_dev, ev ? ev + 6 : nullptr));
       LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 0, cap));
@@ -1248,8 +1291,12 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
   // timing: the cycles that ran
   if (ctx->timing && ctx->pending.size() > pend0 + 4 * (size_t)h.mp_pass) ctx->pending.resize(pend0 + 4 * (size_t)h.mp_pass);
   collect_timing(ctx);
-  if (h.mp_pass > 0) ctx->modal_cycles = h.mp_pass;
   const int it = h.m_iters;
+  if (h.mp_pass > 0) {
+    ctx->modal_cycles = h.mp_pass;
+    // the iterations the whole solve took, a few more: one cycle should do
+    ctx->modal_iters = std::min(NSX_MB_ITERS, std::max(8, it + 4));
+  }
   if (h.exit_code == NSX_SOLVE_MAX_ITERS || h.exit_code == NSX_SOLVE_BREAKDOWN)
     return finish_fp64(ctx, rhs, x, it, h.mp_pass);
   LAUNCH(launch_gnorm_apply(g, s, x, ctx->st_dev));

@@ -210,7 +210,8 @@ int launch_gnorm_sum(const Geo &g, hipStream_t s, const double *x, Partials part
 // Phi^T r), r = b - A x, the stopping rule.  ev: null, or the dispatch's start and stop
 int launch_modal_fwd(const Geo &g, hipStream_t s, const ModalDev &M, const double *r, SolverState *st,
                      hipEvent_t *ev);
-int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, hipEvent_t *ev);
+// (iters: the most iterations of the batched form)
+int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int iters, hipEvent_t *ev);
 int launch_modal_bwd(const Geo &g, hipStream_t s, const ModalDev &M, double *x, SolverState *st, hipEvent_t *ev);
 int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, const double *x, double *r, Partials part,
                       const SolverState *st, hipEvent_t *ev);

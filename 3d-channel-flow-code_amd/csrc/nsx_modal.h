@@ -14,10 +14,27 @@
 // damping of the columns' Jacobi sweeps and of the prolongation's smoothing
 #define NSX_MODAL_OMEGA 0.8f
 #define NSX_MODAL_POMEGA (2.0 / 3.0)
+// Columns from which the 2D solves run batched over the modes (one launch per
+// sweep over the chip) instead of one block per mode.  A random right-hand
+// side to 1e-13, block per mode against batched, 48 layers: 4,096 columns
+// 0.95 ms against 3.7, 8,192 2.5 against 6.0, 16,384 4.8 against 6.7; 65,536 x 96 layers 13
+// against 7.  16 layers: 16,384 columns 4.5 against 6.1.
+#define NSX_MODAL_BATCH 24576
+// blocks of the batched kernels, and the most iterations of a cycle
+#define NSX_MB_GRID 1024
+#define NSX_MB_MEAN 64
+#define NSX_MB_ITERS 60
 // a sparse matrix's rows in slices of 64 (one wave): entry e of row r at
 // ptr[r / 64] + 64 e + r % 64, every row of a slice padded to the longest
 // (index 0, value 0)
 struct SellHost {
+  int n = 0;
+  std::vector<int> ptr, col;
+  std::vector<float> val;
+};
+
+// a matrix row by row
+struct CsrHost {
   int n = 0;
   std::vector<int> ptr, col;
   std::vector<float> val;
@@ -37,6 +54,7 @@ struct ModalHost {
     std::vector<float> diag, area, sabs;  // L's diagonal, the lumped areas, the sum of |off-diagonals|
     SellHost A;   // off-diagonal entries of L (all levels but the columns)
     SellHost R, P;  // restriction to the next level (rows: its nodes), prolongation from it
+    CsrHost Ac, Rc, Pc;  // the same three row by row (levels 0 and 1)
   };
   std::vector<Level> levels;  // level 0: the N0 columns
   std::vector<float> cinv;    // nzi dense nc x nc inverses of the coarsest level
@@ -55,6 +73,16 @@ struct SellDev {
   const float *val;
 };
 
+struct CsrDev {
+  const int *ptr, *col;
+  const float *val;
+};
+
+// a degree-2 Chebyshev smoother: first = r / (th d), then c1 first + c2 r' / d
+struct Cheb {
+  float ith, c1, c2;
+};
+
 // where a mode's vector lies: LDS (float offset) or the mode's workspace
 struct VecLoc {
   int lds;  // 1: in LDS
@@ -63,9 +91,19 @@ struct VecLoc {
 
 struct ModalLevelDev {
   int n;
-  const float *diag, *area, *sabs;
+  const float *diag, *area;
   SellDev A, R, P;
+  CsrDev Ac, Rc, Pc;
+  const Cheb *cheb;  // per mode (the levels between the first and the last)
   VecLoc y, t, b;  // solution, gathered work vector, right-hand side
+};
+
+// the batched 2D solves' scalars per mode
+struct ModeState {
+  double rr, r0, rho, target, scale, inv;
+  double as;    // alpha x scale
+  float beta;
+  int act;      // still iterating
 };
 
 struct ModalDev {
@@ -90,4 +128,15 @@ struct ModalDev {
   double *ap;          // 16 kt x N0p, A p
   float *work;         // nzi x nwork
   double *part;        // npanel x agrid partial sums of the forward transform
+  // batched form: bh, xh, ap and the vectors below are node-major, rows of mp
+  // modes
+  int batched;
+  int mp;                    // 16 kt
+  float *R, *V, *Z, *W, *P[2];  // the columns' FP32 vectors
+  float *y1, *t1, *b1;       // level 1
+  float *y2, *b2;            // level 2
+  ModeState *ms;             // mp
+  double *rpart;             // NSX_MB_MEAN partial sums of mode 0
+  double *rpart2;            // NSX_MB_GRID x mp partial sums per mode
+  int *nact;                 // per iteration: 1 + the last mode still iterating (0: none)
 };

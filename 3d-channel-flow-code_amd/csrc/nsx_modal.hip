@@ -283,6 +283,10 @@ SellHost to_sell(int n, const std::vector<int> &ptr, const std::vector<int> &col
   return S;
 }
 
+CsrHost to_csr(int n, const std::vector<int> &ptr, const std::vector<int> &col, const std::vector<double> &val) {
+  return {n, ptr, col, std::vector<float>(val.begin(), val.end())};
+}
+
 }  // namespace
 
 int modal_build_host(int N0, int nzi, const int *nbr, const double *ppec, const double *area, const double *tlay,
@@ -382,6 +386,7 @@ int modal_build_host(int N0, int nzi, const int *nbr, const double *ppec, const 
       o.sabs[i] = (float)s;
     }
     if (H.levels.size() > 1) o.A = to_sell(G.n, G.ptr, G.col, G.a);
+    if (H.levels.size() == 2) o.Ac = to_csr(G.n, G.ptr, G.col, G.a);
     if (G.n <= NSX_MODAL_COARSE || (int)H.levels.size() == NSX_MODAL_MAXLEV) break;
     int na = 0;
     const std::vector<int> agg = aggregate(G, na);
@@ -389,6 +394,10 @@ int modal_build_host(int N0, int nzi, const int *nbr, const double *ppec, const 
     const Csr P = smoothed_prolongation(G, agg, na), R = transpose(P);
     o.P = to_sell(P.n, P.ptr, P.col, P.val);
     o.R = to_sell(R.n, R.ptr, R.col, R.val);
+    if (H.levels.size() <= 2) {
+      o.Pc = to_csr(P.n, P.ptr, P.col, P.val);
+      o.Rc = to_csr(R.n, R.ptr, R.col, R.val);
+    }
     G = galerkin(G, P, R);
   }
   // the coarsest level's inverses, one per mode; the Neumann mode (mu = 0, L

@@ -45,7 +45,9 @@ __device__ inline void load_layers(const double *p, int k, int nzi, bool ok, dou
   for (int q = 0; q < 4; ++q) v[q] = (ok && k + q < nzi) ? p[k + q] : 0.0;
 }
 
-template <int MT>
+// NODE: bh is node-major (the batched 2D solves): the operands change places,
+// and so do D's rows and columns
+template <int MT, bool NODE>
 __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const double *r, const SolverState *st) {
   if (st->done) return;
   const int kt = M.kt, nzi = M.nzi, m0 = 16 * MT * (int)blockIdx.y;
@@ -69,9 +71,23 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[(size_t)m * kt * 256 + q], b[q], acc[m], 0, 0, 0);
+          acc[m] = NODE ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[q], a[(size_t)m * kt * 256 + q], acc[m], 0, 0, 0)
+                        : __builtin_amdgcn_mfma_f64_16x16x4f64(a[(size_t)m * kt * 256 + q], b[q], acc[m], 0, 0, 0);
 #pragma unroll
       for (int q = 0; q < 4; ++q) b[q] = bn[q];
+    }
+    if (NODE) {
+      // lanes j: 16 consecutive modes of one column (the padding modes' are 0)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        double *dst = M.bh + (size_t)(16 * tile + gq + 4 * q) * M.mp + m0 + j;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          if (m0 + 16 * m < M.mp) dst[16 * m] = acc[m][q];
+          sum[0] += acc[m][q] * acc[m][q];
+        }
+      }
+      continue;
     }
     // lanes j: 16 consecutive columns of one mode, a 128-byte run
 #pragma unroll
@@ -87,7 +103,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
   write_partials<1, MODAL_TB>(sum, M.part + (size_t)blockIdx.y * gridDim.x);
 }
 
-template <int MT>
+template <int MT, bool NODE>
 __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, double *x, SolverState *st) {
   if (st->done) return;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
@@ -104,14 +120,16 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, doubl
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
     // xh's padding modes and columns are zero
-    const double *src = M.xh + (size_t)(4 * gq) * M.N0p + 16 * tile + j;
+    const double *src = NODE ? M.xh + (size_t)(16 * tile + j) * M.mp + 4 * gq
+                             : M.xh + (size_t)(4 * gq) * M.N0p + 16 * tile + j;
+    const size_t step = NODE ? 1 : M.N0p;
     double a[4], an[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = src[(size_t)q * M.N0p];
+    for (int q = 0; q < 4; ++q) a[q] = src[q * step];
     for (int t = 0; t < kt; ++t) {
       if (t + 1 < kt)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) an[q] = src[(size_t)(16 * (t + 1) + q) * M.N0p];
+        for (int q = 0; q < 4; ++q) an[q] = src[(16 * (t + 1) + q) * step];
       const double *b = tab + ((size_t)t * 64 + lane) * 4;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
@@ -141,10 +159,14 @@ static int launch_transform_t(const Geo &g, hipStream_t s, const ModalDev &M, co
                               SolverState *st, bool fwd, hipEvent_t *ev) {
   const size_t lds = (size_t)MT * M.kt * 256 * sizeof(double);
   const dim3 grid(M.agrid, M.npanel), blk(MODAL_TB);
-  if (fwd)
-    LAUNCH_TIMED(ev, 0, k_modal_fwd<MT>, grid, blk, lds, s, g, M, r, st);
+  if (fwd && M.batched)
+    LAUNCH_TIMED(ev, 0, (k_modal_fwd<MT, true>), grid, blk, lds, s, g, M, r, st);
+  else if (fwd)
+    LAUNCH_TIMED(ev, 0, (k_modal_fwd<MT, false>), grid, blk, lds, s, g, M, r, st);
+  else if (M.batched)
+    LAUNCH_TIMED(ev, 0, (k_modal_bwd<MT, true>), grid, blk, lds, s, g, M, x, st);
   else
-    LAUNCH_TIMED(ev, 0, k_modal_bwd<MT>, grid, blk, lds, s, g, M, x, st);
+    LAUNCH_TIMED(ev, 0, (k_modal_bwd<MT, false>), grid, blk, lds, s, g, M, x, st);
   return (int)hipGetLastError();
 }
 
@@ -226,20 +248,74 @@ __device__ inline double block_sum(double v, double (*sh)[W2], int &turn) {
   return s;
 }
 
-// Chebyshev steps of degree 2 on [lmax/4, lmax]: first = r / (th d), then
-// c1 first + c2 r' / d
-struct Cheb {
-  float ith, c1, c2;
-};
-__device__ inline Cheb cheb_of(float lmax) {
-  const float th = 0.625f * lmax, de = 0.375f * lmax, rho0 = de / th, rho1 = 1.f / (2.f * th / de - rho0);
-  return {1.f / th, rho1 * rho0, 2.f * rho1 / de};
+// the V-cycle from level l0 >= 1 down and back up to its solution y, for one
+// mode; on entry the level's right-hand side b, its vector t holding the
+// first Chebyshev step b / (th d) (l0 not the coarsest), with a barrier since
+__device__ inline void cycle_below(const ModalDev &M, int m, float mu, float *work, int l0) {
+  const int tid = threadIdx.x, L = M.nlev;
+  for (int l = l0; l + 1 < L; ++l) {
+    const ModalLevelDev &A = M.lev[l], &C = M.lev[l + 1];
+    const Vec b = vec_at(A.b, work), t = vec_at(A.t, work), y = vec_at(A.y, work), bc = vec_at(C.b, work),
+              tc = vec_at(C.t, work);
+    const Cheb c = A.cheb[m];
+    for (int i = tid; i < A.n; i += T2) {
+      const float d = fmaf(mu, A.area[i], A.diag[i]), t0 = vget(t, i);
+      const float r1 = vget(b, i) - d * t0 - sell_row(A.A, t, i);
+      vset(y, i, t0 + c.c1 * t0 + c.c2 * r1 / d);
+    }
+    __syncthreads();
+    for (int i = tid; i < A.n; i += T2) {
+      const float d = fmaf(mu, A.area[i], A.diag[i]);
+      vset(t, i, vget(b, i) - d * vget(y, i) - sell_row(A.A, y, i));
+    }
+    __syncthreads();
+    const bool last = l + 2 == L;
+    const float ith = last ? 0.f : C.cheb[m].ith;
+    for (int i = tid; i < C.n; i += T2) {
+      const float v = sell_row(A.R, t, i);
+      vset(bc, i, v);
+      if (!last) vset(tc, i, v * ith / fmaf(mu, C.area[i], C.diag[i]));
+    }
+    __syncthreads();
+  }
+  // the coarsest level: eight lanes per row
+  {
+    const ModalLevelDev &A = M.lev[L - 1];
+    const Vec b = vec_at(A.b, work), y = vec_at(A.y, work);
+    const float *ci = M.cinv + (size_t)m * M.nc * M.nc;
+    for (int i0 = 0; i0 < M.nc; i0 += T2 / 8) {
+      const int i = i0 + (tid >> 3);
+      float a = 0.f;
+      if (i < M.nc)
+        for (int k = tid & 7; k < M.nc; k += 8) a = fmaf(ci[(size_t)i * M.nc + k], vget(b, k), a);
+      a += __shfl_xor(a, 4, 64);
+      a += __shfl_xor(a, 2, 64);
+      a += __shfl_xor(a, 1, 64);
+      if (i < M.nc && (tid & 7) == 0) vset(y, i, a);
+    }
+    __syncthreads();
+  }
+  for (int l = L - 2; l >= l0; --l) {
+    const ModalLevelDev &A = M.lev[l];
+    const Vec yc = vec_at(M.lev[l + 1].y, work), b = vec_at(A.b, work), t = vec_at(A.t, work), y = vec_at(A.y, work);
+    const Cheb c = A.cheb[m];
+    for (int i = tid; i < A.n; i += T2) vset(y, i, vget(y, i) + sell_row(A.P, yc, i));
+    __syncthreads();
+    for (int i = tid; i < A.n; i += T2) {
+      const float d = fmaf(mu, A.area[i], A.diag[i]);
+      const float r2 = vget(b, i) - d * vget(y, i) - sell_row(A.A, y, i);
+      vset(b, i, r2);
+      vset(t, i, r2 * c.ith / d);
+    }
+    __syncthreads();
+    for (int i = tid; i < A.n; i += T2) {
+      const float d = fmaf(mu, A.area[i], A.diag[i]), t0 = vget(t, i);
+      const float r3 = vget(b, i) - d * t0 - sell_row(A.A, t, i);
+      vset(y, i, vget(y, i) + t0 + c.c1 * t0 + c.c2 * r3 / d);
+    }
+    __syncthreads();
+  }
 }
-
-struct Lvl {
-  Vec y, t, b;
-  Cheb c;
-};
 
 struct V3 {
   int a, b, c;
@@ -248,7 +324,6 @@ struct V3 {
 __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
   if (st->done) return;
   __shared__ double sh[2][W2];
-  __shared__ Cheb cheb[NSX_MODAL_MAXLEV];
   int turn = 0;
   const int m = blockIdx.x, tid = threadIdx.x, N0 = M.N0, L = M.nlev;
   const double mu64 = M.mu[m];
@@ -278,25 +353,6 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
     return;
   }
   const double scale = sqrt(r0), inv = 1.0 / scale;
-
-  // this mode's Gershgorin bounds on the levels between
-  __syncthreads();
-  for (int l = 1; l + 1 < L; ++l) {
-    const ModalLevelDev &A = M.lev[l];
-    float b = 1.f;
-    for (int i = tid; i < A.n; i += T2) b = fmaxf(b, 1.f + A.sabs[i] / fmaf(mu, A.area[i], A.diag[i]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) b = fmaxf(b, __shfl_xor(b, o, 64));
-    __syncthreads();
-    if ((tid & 63) == 0) sh[0][tid >> 6] = b;
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < W2; ++w) b = fmaxf(b, (float)sh[0][w]);
-      cheb[l] = cheb_of(b);
-    }
-  }
-  __syncthreads();
-  turn = 0;
 
   const Vec V = vec_at(M.lev[0].y, work), Z = vec_at(M.z0, work);
   Vec P0 = vec_at(M.p[0], work), P1 = vec_at(M.p[1], work);
@@ -337,71 +393,18 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
         vset(Z, i, a);
       }
       __syncthreads();
-      // down
-      for (int l = 1; l < L; ++l) {
-        const ModalLevelDev &F = M.lev[l - 1], &A = M.lev[l];
-        const Vec src = l == 1 ? Z : vec_at(F.t, work), b = vec_at(A.b, work), t = vec_at(A.t, work),
-                  y = vec_at(A.y, work);
-        const bool last = l == L - 1;
-        const Cheb c = cheb[last ? 1 : l];
-        for (int i = tid; i < A.n; i += T2) {
-          const float v = sell_row(F.R, src, i);
-          vset(b, i, v);
-          if (!last) vset(t, i, v * c.ith / fmaf(mu, A.area[i], A.diag[i]));
-        }
-        __syncthreads();
-        if (last) break;
-        for (int i = tid; i < A.n; i += T2) {
-          const float d = fmaf(mu, A.area[i], A.diag[i]), t0 = vget(t, i);
-          const float r1 = vget(b, i) - d * t0 - sell_row(A.A, t, i);
-          vset(y, i, t0 + c.c1 * t0 + c.c2 * r1 / d);
-        }
-        __syncthreads();
-        for (int i = tid; i < A.n; i += T2) {
-          const float d = fmaf(mu, A.area[i], A.diag[i]);
-          vset(t, i, vget(b, i) - d * vget(y, i) - sell_row(A.A, y, i));
-        }
-        __syncthreads();
-      }
-      // the coarsest level: eight lanes per row
       {
-        const ModalLevelDev &A = M.lev[L - 1];
-        const Vec b = vec_at(A.b, work), y = vec_at(A.y, work);
-        const float *ci = M.cinv + (size_t)m * M.nc * M.nc;
-        for (int i0 = 0; i0 < M.nc; i0 += T2 / 8) {
-          const int i = i0 + (tid >> 3);
-          float a = 0.f;
-          if (i < M.nc)
-            for (int k = tid & 7; k < M.nc; k += 8) a = fmaf(ci[(size_t)i * M.nc + k], vget(b, k), a);
-          a += __shfl_xor(a, 4, 64);
-          a += __shfl_xor(a, 2, 64);
-          a += __shfl_xor(a, 1, 64);
-          if (i < M.nc && (tid & 7) == 0) vset(y, i, a);
+        const ModalLevelDev &C = M.lev[1];
+        const Vec bc = vec_at(C.b, work), tc = vec_at(C.t, work);
+        const float ith = L == 2 ? 0.f : C.cheb[m].ith;
+        for (int i = tid; i < C.n; i += T2) {
+          const float v = sell_row(M.lev[0].R, Z, i);
+          vset(bc, i, v);
+          if (L > 2) vset(tc, i, v * ith / fmaf(mu, C.area[i], C.diag[i]));
         }
         __syncthreads();
       }
-      // up
-      for (int l = L - 2; l >= 1; --l) {
-        const ModalLevelDev &A = M.lev[l];
-        const Vec yc = vec_at(M.lev[l + 1].y, work), b = vec_at(A.b, work), t = vec_at(A.t, work),
-                  y = vec_at(A.y, work);
-        const Cheb c = cheb[l];
-        for (int i = tid; i < A.n; i += T2) vset(y, i, vget(y, i) + sell_row(A.P, yc, i));
-        __syncthreads();
-        for (int i = tid; i < A.n; i += T2) {
-          const float d = fmaf(mu, A.area[i], A.diag[i]);
-          const float r2 = vget(b, i) - d * vget(y, i) - sell_row(A.A, y, i);
-          vset(b, i, r2);
-          vset(t, i, r2 * c.ith / d);
-        }
-        __syncthreads();
-        for (int i = tid; i < A.n; i += T2) {
-          const float d = fmaf(mu, A.area[i], A.diag[i]), t0 = vget(t, i);
-          const float r3 = vget(b, i) - d * t0 - sell_row(A.A, t, i);
-          vset(y, i, vget(y, i) + t0 + c.c1 * t0 + c.c2 * r3 / d);
-        }
-        __syncthreads();
-      }
+      cycle_below(M, m, mu, work, 1);
       {
         const Vec y1 = vec_at(M.lev[1].y, work);
         for (int i = tid; i < N0; i += T2) vset(V, i, vget(V, i) + sell_row(M.lev[0].P, y1, i));
@@ -479,12 +482,480 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
   if (tid == 0) atomicMax(&st->m_cyc, it);
 }
 
+// --- the 2D solves batched over the modes, for meshes whose vectors pass the
+// LDS.  The same CG and V-cycle on node-major arrays (rows of mp modes), one
+// launch per sweep over the chip: a thread holds four modes of a node, so the
+// graph's indices and weights are read once for all modes (one block per mode
+// reads them per mode, and is bound by its CU's address unit: 500 us an
+// iteration at 65,536 columns x 96 layers, against 190 on average here).  The columns' smoother is
+// the Chebyshev one too, on the mode's own bounds: the high modes, most of the
+// work, take 6 to 11 iterations for 1e-10 instead of 11 to 17, for two more sweeps.
+// Levels 2 and below run one block per mode in LDS.  Modes whose residual has
+// met its target stop; the rows are swept up to the last mode still
+// iterating.  At 6.3M prisms with all modes iterating the update moves 350 MB
+// in 75 us (4.6 TB/s) and the product 126 MB and its gathers in 46 us; with few modes the 20
+// launches' latency bounds the iteration.
+constexpr int MB = NSX_BLOCK;
+
+// f(node, q, K) over the nodes and the groups q of four modes below nact; a
+// thread keeps its q, so what depends on the modes alone (K = make(q)) is
+// read once; blocks take contiguous runs of nodes, an XCD's blocks adjacent
+// ones
+template <class K, class F>
+__device__ inline void mb_nodes(int n, int nact, K &&make, F &&f) {
+  const int n4 = (nact + 3) >> 2, nper = MB / n4, q = threadIdx.x % n4, row = threadIdx.x / n4;
+  const int ng = (n + nper - 1) / nper, G = gridDim.x, b = blockIdx.x;
+  const int lb = (G % NSX_NXCD) == 0 ? (b % NSX_NXCD) * (G / NSX_NXCD) + b / NSX_NXCD : b;
+  const int per = (ng + G - 1) / G, g0 = lb * per, g1 = g0 + per < ng ? g0 + per : ng;
+  if (row >= nper || g0 >= g1) return;
+  const auto k = make(q);
+  for (int g = g0; g < g1; ++g) {
+    const int i = g * nper + row;
+    if (i < n) f(i, q, k);
+  }
+}
+
+struct F4 {
+  float v[4];
+};
+__device__ inline F4 ldf(const float *p) {
+  const float4 a = *(const float4 *)p;
+  return {{a.x, a.y, a.z, a.w}};
+}
+__device__ inline void stf(float *p, const F4 &a) { *(float4 *)p = make_float4(a.v[0], a.v[1], a.v[2], a.v[3]); }
+
+// sum over row i of a CSR matrix times the node-major x
+__device__ inline F4 csr_row(const CsrDev &A, const float *x, int mp, int i, int q) {
+  F4 s = {{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 2
+  for (int e = A.ptr[i]; e < A.ptr[i + 1]; ++e) {
+    const float w = A.val[e];
+    const F4 a = ldf(x + (size_t)A.col[e] * mp + 4 * q);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s.v[k] = fmaf(w, a.v[k], s.v[k]);
+  }
+  return s;
+}
+
+// per-mode sums of a block: thread (row, q) adds acc to mode 4 q + k; row by
+// row in order, so the sums are the same in every run
+__device__ inline void mb_partials(const ModalDev &M, double *P, const double (&acc)[4], int nact) {
+  __shared__ double sh[MB][4];
+  const int n4 = (nact + 3) >> 2, nper = MB / n4;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) sh[threadIdx.x][k] = acc[k];
+  __syncthreads();
+  for (int m = threadIdx.x; m < 4 * n4; m += MB) {
+    double s = 0.0;
+    for (int r = 0; r < nper; ++r) s += sh[r * n4 + (m >> 2)][m & 3];
+    P[(size_t)blockIdx.x * M.mp + m] = s;
+  }
+}
+
+// the sum of mode 0 (its null space is the constants: the mean that rounding
+// leaves in it is no part of the problem)
+__global__ __launch_bounds__(MB) void k_mb_mean(ModalDev M, const SolverState *st) {
+  if (st->done) return;
+  double s[1] = {0.0};
+  for (int i = blockIdx.x * MB + threadIdx.x; i < M.N0; i += gridDim.x * MB) s[0] += M.bh[(size_t)i * M.mp];
+  write_partials<1>(s, M.rpart);
+}
+
+// |r_m|^2 of every mode, mode 0 without its mean
+__global__ __launch_bounds__(MB) void k_mb_norm(ModalDev M, const SolverState *st) {
+  if (st->done) return;
+  double mean[1];
+  reduce_partials<1>(M.rpart, NSX_MB_MEAN, mean);
+  __syncthreads();
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  const double m0 = mean[0] / M.N0;
+  mb_nodes(M.N0, M.mp, [](int) { return 0; }, [&](int i, int q, int) {
+    double r[4];
+    double *p = M.bh + (size_t)i * M.mp + 4 * q;
+    ld4(p, r);
+    if (q == 0) {
+      r[0] -= m0;
+      p[0] = r[0];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] += r[k] * r[k];
+  });
+  mb_partials(M, M.rpart2, acc, M.mp);
+}
+
+// The scalars of 16 modes per block from the partial sums of the kernel
+// before.  WHAT 0: the start (targets, scales); 1: rho and beta; 2: alpha;
+// 3: |r|^2 and which modes go on (nact of iteration it + 1)
+template <int WHAT>
+__global__ __launch_bounds__(T2) void k_mb_scalars(ModalDev M, SolverState *st, int it) {
+  if (st->done) return;
+  const int cur = WHAT == 0 ? M.mp : M.nact[it];
+  if (cur == 0) return;
+  // 64 slices of the rows, 16 modes each
+  __shared__ double sh[T2 / 16][17], shw[2][W2];
+  const int j = threadIdx.x & 15, sl = threadIdx.x >> 4, m = 16 * (int)blockIdx.x + j;
+  double s = 0.0;
+  if (m < cur)
+#pragma unroll 8
+    for (int b = sl; b < NSX_MB_GRID; b += T2 / 16) s += M.rpart2[(size_t)b * M.mp + m];
+  sh[sl][j] = s;
+  double total = 0.0;
+  if (WHAT == 0) {
+    int turn = 0;
+    double tp = 0.0;
+    for (int q = threadIdx.x; q < M.agrid * M.npanel; q += T2) tp += M.part[q];
+    total = block_sum(tp, shw, turn);
+  } else {
+    __syncthreads();
+  }
+  if (sl != 0 || m >= cur) return;
+  s = 0.0;
+  for (int w = 0; w < T2 / 16; ++w) s += sh[w][j];
+  ModeState &S = M.ms[m];
+  if (WHAT == 0) {
+    const double target = st->m_tau * st->m_tau * total / M.nzi;
+    S.rr = S.r0 = s;
+    S.target = target;
+    S.act = s > target && isfinite(s);
+    S.scale = S.act ? sqrt(s) : 1.0;
+    S.inv = 1.0 / S.scale;
+    S.as = 0.0;
+    S.beta = 0.f;
+    if (S.act) atomicMax(&M.nact[0], m + 1);
+  } else if (WHAT == 1) {
+    S.beta = S.act && it > 0 ? (float)(s / S.rho) : 0.f;
+    S.rho = s;
+  } else if (WHAT == 2) {
+    const double alpha = S.rho / s;
+    if (S.act && !(s > 0.0 && isfinite(alpha))) S.act = 0;
+    S.as = S.act ? alpha * S.scale : 0.0;
+  } else {
+    S.rr = s;
+    S.act = S.act && s > S.target;
+    if (S.act) atomicMax(&M.nact[it + 1], m + 1);
+    if (m == 0) st->m_cyc = it + 1;
+  }
+}
+
+__global__ void k_mb_clear(ModalDev M, const SolverState *st) {
+  if (st->done) return;
+  for (int q = threadIdx.x; q <= NSX_MB_ITERS; q += blockDim.x) M.nact[q] = 0;
+}
+
+struct FourCheb {
+  float mu[4];
+  Cheb c[4];
+};
+__device__ inline FourCheb four_cheb(const ModalDev &M, const ModalLevelDev &A, int q) {
+  FourCheb k;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    k.mu[c] = (float)M.mu[4 * q + c];
+    k.c[c] = A.cheb[4 * q + c];
+  }
+  return k;
+}
+
+// x += alpha p, r -= alpha A p, |r|^2, the V-cycle's right-hand side R = r /
+// scale and its first Chebyshev step V = R / (th d) (first: x = 0 and those)
+template <bool FIRST>
+__global__ __launch_bounds__(MB) void k_mb_update(ModalDev M, const float *p, const SolverState *st, int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (!FIRST && nact == 0) return;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  const float *dg = M.lev[0].diag, *ar = M.lev[0].area;
+  struct Kon {
+    float mu[4], ith[4];
+    double inv[4], as[4];
+  };
+  auto make = [&](int q) {
+    Kon k;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      k.mu[c] = (float)M.mu[4 * q + c];
+      k.ith[c] = M.lev[0].cheb[4 * q + c].ith;
+      k.inv[c] = M.ms[4 * q + c].inv;
+      k.as[c] = M.ms[4 * q + c].as;
+    }
+    return k;
+  };
+  mb_nodes(M.N0, FIRST ? mp : nact, make, [&](int i, int q, const Kon &K) {
+    const size_t s = (size_t)i * mp + 4 * q;
+    double r[4], x[4] = {0.0, 0.0, 0.0, 0.0};
+    ld4(M.bh + s, r);
+    if (!FIRST) {
+      double a[4];
+      ld4(M.xh + s, x);
+      ld4(M.ap + s, a);
+      const F4 pv = ldf(p + s);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        x[k] += K.as[k] * (double)pv.v[k];
+        r[k] -= K.as[k] * a[k];
+        acc[k] += r[k] * r[k];
+      }
+      st4(M.bh + s, r);
+    }
+    st4(M.xh + s, x);
+    const float d0 = dg[i], a0 = ar[i];
+    F4 rs, v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      rs.v[k] = (float)(r[k] * K.inv[k]);
+      v.v[k] = rs.v[k] * K.ith[k] / fmaf(K.mu[k], a0, d0);
+    }
+    stf(M.R + s, rs);
+    stf(M.V + s, v);
+  });
+  if (!FIRST) mb_partials(M, M.rpart2, acc, nact);
+}
+
+// the columns' sweeps, as k_mb_smooth's on level 1.  WHAT 0: Z = the Chebyshev
+// sweep from zero (V holds its first step); 1: V = R - A Z; 2: W = R - A Z, V
+// = the first step on it; 3: z = Z + the sweep's rest, partial <r, z>
+template <int WHAT>
+__global__ __launch_bounds__(MB) void k_mb_columns(ModalDev M, const SolverState *st, int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (nact == 0) return;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  auto make = [&](int q) { return four_cheb(M, M.lev[0], q); };
+  mb_nodes(M.N0, nact, make, [&](int i, int q, const FourCheb &K) {
+    const size_t s = (size_t)i * mp + 4 * q;
+    constexpr bool ON_V = WHAT == 0 || WHAT == 3;  // A applied to V, else to Z
+    const float *src = ON_V ? M.V : M.Z;
+    const V3 n = reinterpret_cast<const V3 *>(M.nb)[i];
+    const float4 w = M.wa[i];
+    const F4 c = ldf(src + s), a0 = ldf(src + (size_t)n.a * mp + 4 * q), a1 = ldf(src + (size_t)n.b * mp + 4 * q),
+             a2 = ldf(src + (size_t)n.c * mp + 4 * q), b = ldf((WHAT == 3 ? M.W : M.R) + s);
+    F4 z, rr, o, o2;
+    if (WHAT == 3) {
+      z = ldf(M.Z + s);
+      rr = ldf(M.R + s);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float d = fmaf(K.mu[k], w.w, w.x + w.y + w.z);
+      const float r = fmaf(w.x, a0.v[k], fmaf(w.y, a1.v[k], fmaf(w.z, a2.v[k], fmaf(-d, c.v[k], b.v[k]))));
+      o.v[k] = r;
+      if (ON_V) o.v[k] = (WHAT == 3 ? z.v[k] : 0.f) + c.v[k] + K.c[k].c1 * c.v[k] + K.c[k].c2 * r / d;
+      if (WHAT == 2) o2.v[k] = r * K.c[k].ith / d;
+      if (WHAT == 3) acc[k] += (double)rr.v[k] * (double)o.v[k];
+    }
+    stf((ON_V ? M.Z : WHAT == 1 ? M.V : M.W) + s, o);
+    if (WHAT == 2) stf(M.V + s, o2);
+  });
+  if (WHAT == 3) mb_partials(M, M.rpart2, acc, nact);
+}
+
+// p = z + beta p_old at the column and its neighbours, A p in FP64, <p, A p>
+__global__ __launch_bounds__(MB) void k_mb_ap(ModalDev M, const float *pold, float *pnew, const SolverState *st,
+                                              int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (nact == 0) return;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  struct Kon {
+    float beta[4];
+    double mu[4];
+  };
+  auto make = [&](int q) {
+    Kon k;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      k.beta[c] = M.ms[4 * q + c].beta;
+      k.mu[c] = M.mu[4 * q + c];
+    }
+    return k;
+  };
+  mb_nodes(M.N0, nact, make, [&](int i, int q, const Kon &K) {
+    const V3 n = reinterpret_cast<const V3 *>(M.nb)[i];
+    const double *w = M.w64 + 3 * (size_t)i;
+    const int id[4] = {i, n.a, n.b, n.c};
+    F4 p[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const size_t s = (size_t)id[c] * mp + 4 * q;
+      p[c] = ldf(M.Z + s);
+      if (it > 0) {
+        const F4 o = ldf(pold + s);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[c].v[k] = fmaf(K.beta[k], o.v[k], p[c].v[k]);
+      }
+    }
+    const double w0 = w[0], w1 = w[1], w2 = w[2], ar = M.area64[i];
+    double a[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double pd = (double)p[0].v[k];
+      a[k] = w0 * (pd - (double)p[1].v[k]) + w1 * (pd - (double)p[2].v[k]) + w2 * (pd - (double)p[3].v[k]) +
+             K.mu[k] * ar * pd;
+      acc[k] += pd * a[k];
+    }
+    const size_t s = (size_t)i * mp + 4 * q;
+    stf(pnew + s, p[0]);
+    st4(M.ap + s, a);
+  });
+  mb_partials(M, M.rpart2, acc, nact);
+}
+
+// b of the level below = R src, and (t not null) its first Chebyshev step
+__global__ __launch_bounds__(MB) void k_mb_restrict(ModalDev M, CsrDev R, int lc, const float *src, float *b, float *t,
+                                                    const SolverState *st, int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (nact == 0) return;
+  const ModalLevelDev &C = M.lev[lc];
+  struct Kon {
+    float mu[4], ith[4];
+  };
+  auto make = [&](int q) {
+    Kon k;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      k.mu[c] = (float)M.mu[4 * q + c];
+      k.ith[c] = t ? C.cheb[4 * q + c].ith : 0.f;
+    }
+    return k;
+  };
+  mb_nodes(C.n, nact, make, [&](int i, int q, const Kon &K) {
+    const size_t s = (size_t)i * mp + 4 * q;
+    const F4 v = csr_row(R, src, mp, i, q);
+    stf(b + s, v);
+    if (t) {
+      const float dg = C.diag[i], ar = C.area[i];
+      F4 o;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o.v[k] = v.v[k] * K.ith[k] / fmaf(K.mu[k], ar, dg);
+      stf(t + s, o);
+    }
+  });
+}
+
+__global__ __launch_bounds__(MB) void k_mb_prolong(ModalDev M, CsrDev P, int n, const float *yc, float *y,
+                                                   const SolverState *st, int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (nact == 0) return;
+  mb_nodes(n, nact, [](int) { return 0; }, [&](int i, int q, int) {
+    const size_t s = (size_t)i * mp + 4 * q;
+    const F4 a = csr_row(P, yc, mp, i, q);
+    F4 v = ldf(y + s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v.v[k] += a.v[k];
+    stf(y + s, v);
+  });
+}
+
+// level 1's sweeps.  WHAT 0: y = the Chebyshev sweep from zero (t holds its
+// first step); 1: t = b - A y; 2: b = b - A y, t = the first step on it;
+// 3: y += the sweep's rest
+template <int WHAT>
+__global__ __launch_bounds__(MB) void k_mb_smooth(ModalDev M, const SolverState *st, int it) {
+  if (st->done) return;
+  const int nact = M.nact[it], mp = M.mp;
+  if (nact == 0) return;
+  const ModalLevelDev &A = M.lev[1];
+  auto make = [&](int q) { return four_cheb(M, A, q); };
+  mb_nodes(A.n, nact, make, [&](int i, int q, const FourCheb &K) {
+    const size_t s = (size_t)i * mp + 4 * q;
+    constexpr bool ON_T = WHAT == 0 || WHAT == 3;  // A applied to t, else to y
+    const float *src = ON_T ? M.t1 : M.y1;
+    const F4 a = csr_row(A.Ac, src, mp, i, q), c = ldf(src + s), b = ldf(M.b1 + s);
+    const float dg = A.diag[i], ar = A.area[i];
+    F4 y, o, o2;
+    if (WHAT == 3) y = ldf(M.y1 + s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const Cheb h = K.c[k];
+      const float d = fmaf(K.mu[k], ar, dg), r = b.v[k] - d * c.v[k] - a.v[k];
+      o.v[k] = r;
+      if (ON_T) o.v[k] = (WHAT == 3 ? y.v[k] : 0.f) + c.v[k] + h.c1 * c.v[k] + h.c2 * r / d;
+      if (WHAT == 2) o2.v[k] = r * h.ith / d;
+    }
+    stf((ON_T ? M.y1 : WHAT == 1 ? M.t1 : M.b1) + s, o);
+    if (WHAT == 2) stf(M.t1 + s, o2);
+  });
+}
+
+// levels 2 and below, a block per mode
+__global__ __launch_bounds__(T2) void k_mb_below(ModalDev M, const SolverState *st, int it) {
+  if (st->done) return;
+  const int m = blockIdx.x, mp = M.mp, tid = threadIdx.x;
+  if (m >= M.nact[it] || !M.ms[m].act) return;
+  const ModalLevelDev &A = M.lev[2];
+  float *work = M.work + (size_t)m * M.nwork;
+  const float mu = (float)M.mu[m];
+  const Vec b = vec_at(A.b, work), t = vec_at(A.t, work), y = vec_at(A.y, work);
+  const bool last = M.nlev == 3;
+  const float ith = last ? 0.f : A.cheb[m].ith;
+  for (int i = tid; i < A.n; i += T2) {
+    const float v = M.b2[(size_t)i * mp + m];
+    vset(b, i, v);
+    if (!last) vset(t, i, v * ith / fmaf(mu, A.area[i], A.diag[i]));
+  }
+  __syncthreads();
+  cycle_below(M, m, mu, work, 2);
+  for (int i = tid; i < A.n; i += T2) M.y2[(size_t)i * mp + m] = vget(y, i);
+}
+
+// no correction from a mode whose solve gained nothing
+__global__ __launch_bounds__(MB) void k_mb_final(ModalDev M, const SolverState *st) {
+  if (st->done) return;
+  bool any = false;
+  for (int m = 0; m < M.nzi; ++m) any = any || !(M.ms[m].rr <= M.ms[m].r0);
+  if (!any) return;
+  for (size_t s = (size_t)blockIdx.x * MB + threadIdx.x; s < (size_t)M.N0 * M.mp; s += (size_t)gridDim.x * MB) {
+    const ModeState &S = M.ms[s % M.mp];
+    if (!(S.rr <= S.r0)) M.xh[s] = 0.0;
+  }
+}
+
+static int launch_batched(hipStream_t s, const ModalDev &M, SolverState *st, int iters) {
+  const dim3 grid(NSX_MB_GRID), blk(MB), sc(M.kt);
+  hipLaunchKernelGGL(k_mb_clear, dim3(1), dim3(64), 0, s, M, st);
+  hipLaunchKernelGGL(k_mb_mean, dim3(NSX_MB_MEAN), blk, 0, s, M, st);
+  hipLaunchKernelGGL(k_mb_norm, grid, blk, 0, s, M, st);
+  hipLaunchKernelGGL(k_mb_scalars<0>, sc, dim3(T2), 0, s, M, st, 0);
+  hipLaunchKernelGGL(k_mb_update<true>, grid, blk, 0, s, M, (const float *)nullptr, st, 0);
+  const ModalLevelDev &C = M.lev[0], &A = M.lev[1];
+  for (int it = 0; it < iters && it < NSX_MB_ITERS; ++it) {
+    hipLaunchKernelGGL(k_mb_columns<0>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_columns<1>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_restrict, grid, blk, 0, s, M, C.Rc, 1, (const float *)M.V, M.b1, M.t1, st, it);
+    hipLaunchKernelGGL(k_mb_smooth<0>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_smooth<1>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_restrict, grid, blk, 0, s, M, A.Rc, 2, (const float *)M.t1, M.b2, (float *)nullptr, st, it);
+    hipLaunchKernelGGL(k_mb_below, dim3(M.nzi), dim3(T2), (size_t)M.lds2d, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_prolong, grid, blk, 0, s, M, A.Pc, A.n, (const float *)M.y2, M.y1, st, it);
+    hipLaunchKernelGGL(k_mb_smooth<2>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_smooth<3>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_prolong, grid, blk, 0, s, M, C.Pc, M.N0, (const float *)M.y1, M.Z, st, it);
+    hipLaunchKernelGGL(k_mb_columns<2>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_columns<3>, grid, blk, 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_scalars<1>, sc, dim3(T2), 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_ap, grid, blk, 0, s, M, (const float *)M.P[it & 1], M.P[(it + 1) & 1], st, it);
+    hipLaunchKernelGGL(k_mb_scalars<2>, sc, dim3(T2), 0, s, M, st, it);
+    hipLaunchKernelGGL(k_mb_update<false>, grid, blk, 0, s, M, (const float *)M.P[(it + 1) & 1], st, it);
+    hipLaunchKernelGGL(k_mb_scalars<3>, sc, dim3(T2), 0, s, M, st, it);
+  }
+  hipLaunchKernelGGL(k_mb_final, grid, blk, 0, s, M, st);
+  return (int)hipGetLastError();
+}
+
 int launch_modal_fwd(const Geo &g, hipStream_t s, const ModalDev &M, const double *r, SolverState *st,
                      hipEvent_t *ev) {
   return launch_transform(g, s, M, r, nullptr, st, true, ev);
 }
 
-int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, hipEvent_t *ev) {
+int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int iters, hipEvent_t *ev) {
+  if (M.batched) {
+    if (ev) (void)hipEventRecord(ev[0], s);
+    const int rc = launch_batched(s, M, st, iters);
+    if (ev) (void)hipEventRecord(ev[1], s);
+    return rc;
+  }
   LAUNCH_TIMED(ev, 0, k_modal_2d, dim3(M.nzi), dim3(T2), (size_t)M.lds2d, s, M, st);
   return (int)hipGetLastError();
 }
@@ -493,19 +964,23 @@ int launch_modal_bwd(const Geo &g, hipStream_t s, const ModalDev &M, double *x, 
   return launch_transform(g, s, M, nullptr, x, st, false, ev);
 }
 
+static bool allow(const void *kern, int lds) {
+  return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+}
+
 template <int MT>
 static bool allow_t(int lds) {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_modal_fwd<MT>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess &&
-         hipFuncSetAttribute(reinterpret_cast<const void *>(&k_modal_bwd<MT>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+  return allow(reinterpret_cast<const void *>(&k_modal_fwd<MT, false>), lds) &&
+         allow(reinterpret_cast<const void *>(&k_modal_fwd<MT, true>), lds) &&
+         allow(reinterpret_cast<const void *>(&k_modal_bwd<MT, false>), lds) &&
+         allow(reinterpret_cast<const void *>(&k_modal_bwd<MT, true>), lds);
 }
 
 // raises the kernels' dynamic LDS limits to what M asks for
 bool modal_allow_lds(const ModalDev &M) {
   const int tr = M.mt * M.kt * 256 * (int)sizeof(double);
-  bool ok = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_modal_2d),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, M.lds2d) == hipSuccess;
+  const bool ok = M.batched ? allow(reinterpret_cast<const void *>(&k_mb_below), M.lds2d)
+                            : allow(reinterpret_cast<const void *>(&k_modal_2d), M.lds2d);
   switch (M.mt) {
     case 1: return ok && allow_t<1>(tr);
     case 2: return ok && allow_t<2>(tr);

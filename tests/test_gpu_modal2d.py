@@ -48,14 +48,19 @@ def _check(c, seed):
     (12, 8, 130),    # two panels
     (12, 8, 260),    # seventeen tiles, one past the eight a block accumulates twice over
     (90, 41, 9),     # 7,380 columns: the columns' vectors pass the block's LDS
+    (160, 76, 6),    # 24,320 columns: the most that take a block per mode
+    (160, 77, 6),    # 24,640: batched over the modes, ten of a tile's sixteen unused
+    (201, 79, 17),   # odd columns, one mode past a tile
+    (160, 80, 67),   # five tiles: thread groups that do not divide a block
 ])
 def test_modal_sizes(nx, ny, nn):
     _check(make_case(nx, ny, nn, seed=11, jitter=0.1), seed=nx + nn)
 
 
 @pytest.mark.parametrize("walls", [(1, 0, 0, 0), (0, 0, 0, 0), (0, 1, 1, 1)])
-def test_modal_walls_odd(walls):
-    _check(make_case(27, 15, 19, seed=5, jitter=0.1, walls=walls), seed=3)
+@pytest.mark.parametrize("nx, ny, nn", [(27, 15, 19), (159, 79, 7)])
+def test_modal_walls_odd(nx, ny, nn, walls):
+    _check(make_case(nx, ny, nn, seed=5, jitter=0.1, walls=walls), seed=3)
 
 
 def test_modal_zero_and_solved_right_hand_sides():
