@@ -47,6 +47,19 @@ struct AdjWork {
 
 }  // namespace
 
+// nsx_put_field / nsx_get_field: see xfer_setup
+struct Xfer {
+  bool ready = false;
+  size_t chunk = 0;  // doubles
+  double *pin[2] = {nullptr, nullptr}, *dev[2] = {nullptr, nullptr};
+  hipEvent_t done[2] = {nullptr, nullptr};
+  int nrow = 0, *src = nullptr;  // the ghost rows filled and their device columns
+  std::vector<int> row;
+  bool contiguous = false;       // every ghost row, in order
+};
+// 4 MB: a chunk's crossing (70 us) hides its launches, two stay in the host's cache
+#define NSX_XFER_CHUNK (512 * 1024)
+
 struct nsx_ctx {
   int N0 = 0, NC = 0, NV = 0, NZ = 0, NS = 0, NEX = 0;
   int NGW = 0;                 // wall ghost columns after the N0 interior ones
@@ -118,6 +131,7 @@ struct nsx_ctx {
   std::vector<double> h_ppec;
   ModalDev modal{};
   bool modal_ok = false;
+  Xfer xfer;
   int modal_cycles = 0, modal_iters = 44;
   int iter_hint_cg = 0;
   int iter_hint_cgs = 0;
@@ -217,6 +231,10 @@ extern "C" int nsx_destroy(nsx_ctx *ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   for (void *p : ctx->allocs) (void)hipFree(p);
   if (ctx->st_host) (void)hipHostFree(ctx->st_host);
+  for (int q = 0; q < 2; ++q) {
+    if (ctx->xfer.pin[q]) (void)hipHostFree(ctx->xfer.pin[q]);
+    if (ctx->xfer.done[q]) (void)hipEventDestroy(ctx->xfer.done[q]);
+  }
   for (hipEvent_t ev : ctx->evpool) (void)hipEventDestroy(ev);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -794,55 +812,118 @@ static int check_field(nsx_ctx *ctx, int f) {
   return 0;
 }
 
+// The transfers' buffers, made at the first one: two chunks of layers in
+// pinned host memory and on the device, so that one crosses while the host
+// copies the other, and the ghost rows nsx_get_field fills.
+static int xfer_setup(nsx_ctx *ctx) {
+  Xfer &X = ctx->xfer;
+  if (X.ready) return 0;
+  const int N0 = ctx->N0, NC = ctx->NC;
+  // a periodic ghost row is its partner's column, a wall ghost row the
+  // device's wall ghost column
+  std::vector<int> src;
+  std::vector<int> wall((size_t)(NC - N0) + 1, -1);
+  for (int w = 0; w < ctx->NGW; ++w) wall[ctx->gw_ghost[w] - N0] = N0 + w;
+  X.row.clear();
+  for (int gh = N0; gh < ctx->NEX; ++gh) {
+    const int partner = ctx->No_cp[(size_t)gh + 2 * (size_t)NC] - 1;
+    const int c = wall[gh - N0] >= 0 ? wall[gh - N0] : (partner >= 0 && partner < N0) ? partner : -1;
+    if (c < 0) continue;
+    X.row.push_back(gh);
+    src.push_back(c);
+  }
+  X.nrow = (int)src.size();
+  X.contiguous = X.nrow == ctx->NEX - N0;
+  int rc;
+  if ((rc = dev_upload(ctx, &X.src, src))) return rc;
+  // a chunk holds at least one layer of every kind of field
+  X.chunk = std::max((size_t)NSX_XFER_CHUNK, (size_t)std::max(std::max(ctx->NEX, N0 + ctx->NGW), ctx->NV));
+  for (int q = 0; q < 2; ++q) {
+    if ((rc = dev_alloc(ctx, &X.dev[q], X.chunk))) return rc;
+    HIPCHECK(hipHostMalloc((void **)&X.pin[q], X.chunk * sizeof(double), hipHostMallocDefault));
+    HIPCHECK(hipEventCreateWithFlags(&X.done[q], hipEventDisableTiming));
+  }
+  X.ready = true;
+  return 0;
+}
+
 extern "C" int nsx_put_field(nsx_ctx *ctx, int f, const double *host) {
   NEED_COMMIT(ctx);
   if (check_field(ctx, f)) return -1;
   reset_guess(ctx);  // a new state: the stored solutions no longer lead to it
-  const int N0 = ctx->N0, NZ = ctx->NZ, NS = ctx->NS, NV = ctx->NV;
-  std::vector<double> buf(field_elems(ctx, ctx->kind[f]), 0.0);
-  if (ctx->kind[f] == FK_VERT) {
-    for (int l = 0; l < NZ - 1; ++l)
-      for (int v = 0; v < NV; ++v) buf[(size_t)v * (NZ - 1) + l] = host[(size_t)v + (size_t)l * NV];
-  } else {
-    const size_t ld = ctx->kind[f] == FK_FACE ? (size_t)N0 : (size_t)ctx->NC;
-    for (int k = 0; k < NZ; ++k)
-      for (int i = 0; i < N0; ++i) buf[(size_t)i * NS + k] = host[(size_t)i + (size_t)k * ld];
-    // wall ghost rows are state the caller's BC calls wrote; periodic ghost
-    // rows are not stored (the neighbour index points at the partner)
-    if (ctx->kind[f] == FK_CELL)
-      for (int w = 0; w < ctx->NGW; ++w)
-        for (int k = 0; k < NZ; ++k)
-          buf[(size_t)(N0 + w) * NS + k] = host[(size_t)ctx->gw_ghost[w] + (size_t)k * ld];
+  int rc = xfer_setup(ctx);
+  if (rc) return rc;
+  Xfer &X = ctx->xfer;
+  hipStream_t s = ctx->stream;
+  const int N0 = ctx->N0, kind = ctx->kind[f];
+  const bool vert = kind == FK_VERT;
+  // wall ghost rows are state the caller's BC calls wrote; periodic ghost
+  // rows are not stored (the neighbour index points at the partner)
+  const int ngw = kind == FK_CELL ? ctx->NGW : 0, n = vert ? ctx->NV : N0, w = n + ngw;
+  const size_t ld = vert ? (size_t)ctx->NV : kind == FK_FACE ? (size_t)N0 : (size_t)ctx->NC;
+  const int kz = vert ? ctx->NZ - 1 : ctx->NZ, stride = vert ? ctx->NZ - 1 : ctx->NS;
+  const int step = std::max(1, (int)(X.chunk / (size_t)w));
+  for (int k0 = 0, c = 0; k0 < stride; k0 += step, ++c) {
+    const int nk = std::min(step, stride - k0), q = c & 1;
+    if (c >= 2) HIPCHECK(hipEventSynchronize(X.done[q]));
+    const int nh = std::max(0, std::min(nk, kz - k0));
+    for (int k = 0; k < nh; ++k) {
+      const double *src = host + (size_t)(k0 + k) * ld;
+      double *dst = X.pin[q] + (size_t)k * w;
+      memcpy(dst, src, (size_t)n * sizeof(double));
+      for (int e = 0; e < ngw; ++e) dst[n + e] = src[ctx->gw_ghost[e]];
+    }
+    // a field of one chunk is read from the pinned memory itself: a copy's
+    // set-up costs more than it saves
+    const bool one = step >= stride;
+    if (nh && !one)
+      HIPCHECK(hipMemcpyAsync(X.dev[q], X.pin[q], (size_t)nh * w * sizeof(double), hipMemcpyHostToDevice, s));
+    LAUNCH(launch_field_in(s, one ? X.pin[q] : X.dev[q], w, k0, nk, kz, stride, ctx->slot[f]));
+    if (!one) HIPCHECK(hipEventRecord(X.done[q], s));
   }
-  HIPCHECK(hipMemcpyAsync(ctx->slot[f], buf.data(), buf.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHECK(hipStreamSynchronize(ctx->stream));
+  HIPCHECK(hipStreamSynchronize(s));
   return 0;
 }
 
 extern "C" int nsx_get_field(nsx_ctx *ctx, int f, double *host, int fill_ghost_rows) {
   NEED_COMMIT(ctx);
   if (check_field(ctx, f)) return -1;
-  const int N0 = ctx->N0, NZ = ctx->NZ, NS = ctx->NS, NV = ctx->NV, NC = ctx->NC;
-  std::vector<double> buf(field_elems(ctx, ctx->kind[f]));
-  HIPCHECK(hipMemcpyAsync(buf.data(), ctx->slot[f], buf.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHECK(hipStreamSynchronize(ctx->stream));
-  if (ctx->kind[f] == FK_VERT) {
-    for (int l = 0; l < NZ - 1; ++l)
-      for (int v = 0; v < NV; ++v) host[(size_t)v + (size_t)l * NV] = buf[(size_t)v * (NZ - 1) + l];
+  int rc = xfer_setup(ctx);
+  if (rc) return rc;
+  Xfer &X = ctx->xfer;
+  hipStream_t s = ctx->stream;
+  const int N0 = ctx->N0, kind = ctx->kind[f];
+  const bool vert = kind == FK_VERT, ghosts = fill_ghost_rows && kind == FK_CELL;
+  const int n = vert ? ctx->NV : N0, w = n + (ghosts ? X.nrow : 0);
+  const size_t ld = vert ? (size_t)ctx->NV : kind == FK_FACE ? (size_t)N0 : (size_t)ctx->NC;
+  const int kz = vert ? ctx->NZ - 1 : ctx->NZ, stride = vert ? ctx->NZ - 1 : ctx->NS;
+  const int step = std::max(1, (int)(X.chunk / (size_t)w)), nchunk = (kz + step - 1) / step;
+  auto issue = [&](int c) -> int {
+    const int k0 = c * step, nk = std::min(step, kz - k0), q = c & 1;
+    // one chunk: written to the pinned memory itself (see nsx_put_field)
+    LAUNCH(launch_field_out(s, ctx->slot[f], stride, k0, nk, w, n, X.src, nchunk == 1 ? X.pin[q] : X.dev[q]));
+    if (nchunk == 1) return 0;
+    HIPCHECK(hipMemcpyAsync(X.pin[q], X.dev[q], (size_t)nk * w * sizeof(double), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipEventRecord(X.done[q], s));
     return 0;
-  }
-  const size_t ld = ctx->kind[f] == FK_FACE ? (size_t)N0 : (size_t)NC;
-  for (int k = 0; k < NZ; ++k)
-    for (int i = 0; i < N0; ++i) host[(size_t)i + (size_t)k * ld] = buf[(size_t)i * NS + k];
-  if (fill_ghost_rows && ctx->kind[f] == FK_CELL) {
-    for (int gh = N0; gh < ctx->NEX; ++gh) {
-      const int partner = ctx->No_cp[(size_t)gh + 2 * (size_t)NC] - 1;
-      if (partner < 0 || partner >= N0) continue;
-      for (int k = 0; k < NZ; ++k) host[(size_t)gh + (size_t)k * NC] = buf[(size_t)partner * NS + k];
+  };
+  if ((rc = issue(0))) return rc;
+  for (int c = 0; c < nchunk; ++c) {
+    if (c + 1 < nchunk && (rc = issue(c + 1))) return rc;
+    if (nchunk == 1)
+      HIPCHECK(hipStreamSynchronize(s));
+    else
+      HIPCHECK(hipEventSynchronize(X.done[c & 1]));
+    const int k0 = c * step, nk = std::min(step, kz - k0);
+    for (int k = 0; k < nk; ++k) {
+      const double *src = X.pin[c & 1] + (size_t)k * w;
+      double *dst = host + (size_t)(k0 + k) * ld;
+      // rows that no rule fills stay as the caller left them
+      const bool whole = w == n || X.contiguous;
+      memcpy(dst, src, (size_t)(whole ? w : n) * sizeof(double));
+      if (!whole)
+        for (int e = 0; e < X.nrow; ++e) dst[X.row[e]] = src[n + e];
     }
-    for (int w = 0; w < ctx->NGW; ++w)
-      for (int k = 0; k < NZ; ++k)
-        host[(size_t)ctx->gw_ghost[w] + (size_t)k * NC] = buf[(size_t)(N0 + w) * NS + k];
   }
   return 0;
 }

@@ -127,6 +127,10 @@ int launch_extrapolate(const Geo &g, hipStream_t s, const double *a, const doubl
 int launch_ghost_layers(const Geo &g, hipStream_t s, double *f, int kind /*0 p, 1 u, 2 v, 3 w*/);
 int launch_ppe_diag(const Geo &g, hipStream_t s, double *A0);
 int launch_copy(hipStream_t s, size_t n, const double *src, double *dst);
+// nsx_put_field / nsx_get_field (nsx_xfer.hip)
+int launch_field_out(hipStream_t s, const double *f, int stride, int k0, int nk, int w, int n, const int *ghost,
+                     double *out);
+int launch_field_in(hipStream_t s, const double *in, int w, int k0, int nk, int kz, int stride, double *f);
 // glob_cfl (nsx_diag.hip): partial rows per block, and the 13 outputs into out
 // channel statistics (stats.F90): the twelve accumulators of glob_sample,
 // in the order of module stats; the first nine are glob_put_plane_mm's

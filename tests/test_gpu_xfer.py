@@ -1,0 +1,46 @@
+"""nsx_put_field / nsx_get_field: fields that cross in one chunk of layers, in
+several and in ragged last ones, of every kind, periodic and walled: what
+comes back is what went (bit for bit), periodic ghost rows are their
+partners', rows that no rule fills stay as the caller left them."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from nsx.abi import F
+from nsx.case import make_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx, ny, nn, walls", [
+    (2, 2, 2, None),          # one tile, one chunk
+    (33, 17, 31, (1, 0, 0, 0)),  # odd columns and layers, wall ghost rows
+    (32, 16, 30, None),       # as many layers as a tile
+    (90, 45, 67, None),       # 4.5 MB: two chunks, the last ragged
+    (128, 64, 64, (0, 0, 0, 0)),  # three chunks
+])
+def test_round_trip(nx, ny, nn, walls):
+    from nsx.device import Context
+    c = make_case(nx, ny, nn, seed=3, jitter=0.1, walls=walls)
+    rng = np.random.default_rng(nx)
+    G = Context(c)
+    n0, nex = c.N_CELL0, c.N_CELLexact
+    for name in ("UFN", "EDDY", "UFV", "UTFACE"):
+        shape = G._shape(F[name])
+        a = np.asfortranarray(rng.standard_normal(shape[::-1]).T)
+        G.put(name, a)
+        out = np.full(shape, -7.0, order="F")
+        G._check(G.lib.nsx_get_field(G.h, F[name], ctypes.c_void_p(out.ctypes.data), 0))
+        n = n0 if shape[0] == c.N_CELL else shape[0]
+        assert np.array_equal(out[:n], a[:n]), name
+        assert np.all(out[n:] == -7.0), name
+        if shape[0] != c.N_CELL:
+            continue
+        G._check(G.lib.nsx_get_field(G.h, F[name], ctypes.c_void_p(out.ctypes.data), 1))
+        partner = np.asarray(c.No_cp)[n0:nex, 2] - 1
+        for g in range(n0, nex):
+            wall = c.bcpc[g] == 1
+            assert np.array_equal(out[g], a[g] if wall else a[partner[g - n0]]), (name, g)
+        assert np.all(out[nex:] == -7.0), name
+    G.close()
