@@ -307,8 +307,9 @@ __global__ __launch_bounds__(NSX_BLOCK) void k_bicg_init_state(SolverState *st, 
 // the breakdown guards of :479-490; at k = 0 the norms of :453-469) from C's
 // partial sums (P.init at k = 0).  Returns
 // false when the solve stops; sets beta (0 at k = 0).
+// (pre: C's totals where the caller has summed them already)
 __device__ inline bool begin_iteration(const Geo &g, Partials P, SolverState *st, double &beta_out,
-                                       bool &first_out) {
+                                       bool &first_out, const double *pre = nullptr) {
   const int k_it = st->c_iter;
   const bool first = k_it == 0;
   double rho, e1, e2, xvol, b1, b2;
@@ -336,7 +337,10 @@ __device__ inline bool begin_iteration(const Geo &g, Partials P, SolverState *st
     }
   } else {
     double t[4];
-    reduce_partials<4>(P.c, gridDim.x, t);
+    if (pre)
+      for (int q = 0; q < 4; ++q) t[q] = pre[q];
+    else
+      reduce_partials<4>(P.c, gridDim.x, t);
     b1 = st->b1;
     b2 = st->b2;
     const double r2 = sqrt(t[0]), r1 = t[1];
@@ -732,6 +736,189 @@ __global__ __launch_bounds__(NSX_BLOCK) void k_bicg_c(Geo g, T *x, T *rt, T *q, 
     st4(q + s0, qq);
   });
   write_partials<4>(acc, P.c);
+}
+
+// ------------------------------------------- one window a block -----------
+// Phases A and B on meshes of at most NSX_ONE_WINDOW windows, block b working
+// on window b alone.  Such a launch is bound by its chain of dependent
+// loads, not by bytes: the swept kernels read the stop flag, the scalars,
+// the partial sums, the levels, the neighbours and the vectors one after the
+// other.  Here every load (the partial sums, the levels, the neighbours, the
+// vectors at the window and at its outer neighbours) is issued before the
+// first barrier, which the reduction and the level table share.  The values
+// formed are those of the swept kernels.  A and B, us, before -> after: 36
+// windows 10.9 -> 6.9 and 8.1 -> 5.4 (the grid of 32 blocks took two rounds),
+// 208 windows 8.9 -> 8.0 and 6.5 -> 5.6, 352 windows 10.8 -> 9.1 and 7.4 ->
+// 6.4; at 1,088 windows the swept ones win (the blocks no longer wait alone).
+// Phase C the same way gained nothing (208 windows: 6.6 -> 7.4).
+template <int K>
+__device__ inline void part_load(const double *P, double (&v)[K]) {
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    v[q] = 0.0;
+    for (uint32_t b = threadIdx.x; b < gridDim.x; b += NSX_BLOCK) v[q] += P[(size_t)q * gridDim.x + b];
+  }
+}
+
+// the levels into LDS and the totals of the block's partial sums, one barrier
+template <int K>
+__device__ inline const double *part_levels(const Geo &g, double (&v)[K]) {
+  extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
+  __shared__ double sh[K][NSX_BLOCK / 64];
+  double *lv = reinterpret_cast<double *>(nsx_dyn_lds);
+  for (int k = threadIdx.x; k < g.NS; k += NSX_BLOCK) {
+    lv[k] = k < g.NZ ? g.dsig[k] : 1.0;
+    lv[g.NS + k] = k < g.NZ - 1 ? g.dsigv[k] : 1.0;
+  }
+  wave_sum<K>(v);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < K; ++q) sh[q][threadIdx.x >> 6] = v[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    v[q] = 0.0;
+    for (int w = 0; w < NSX_BLOCK / 64; ++w) v[q] += sh[q][w];
+  }
+  return lv;
+}
+
+template <typename T>
+struct Win {
+  bool act;
+  int i, k0;
+  uint32_t lim, d[3];
+  size_t s0;
+  T a[4], b[4], na[3][4], nb[3][4], am, bm, ap, bp;
+  Col<T> C;
+};
+
+template <typename T>
+__device__ inline void win_load(const Geo &g, const T *a, const T *b, Win<T> &W) {
+  const uint32_t base = blockIdx.x * NSX_BLOCK, end = base + NSX_BLOCK < g.nquad ? base + NSX_BLOCK : g.nquad;
+  const uint32_t t = base + threadIdx.x;
+  W.act = t < end;
+  W.lim = end - base;
+  W.i = 0;
+  W.k0 = 0;
+  W.s0 = 0;
+  W.am = W.bm = W.ap = W.bp = T(0);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) W.a[u] = W.b[u] = T(0);
+  if (!W.act) return;
+  W.i = (int)fdiv(t, g.divNQ);
+  W.k0 = 4 * (int)(t - (uint32_t)W.i * (uint32_t)g.NQ);
+  W.s0 = (size_t)W.i * g.NS + W.k0;
+  int n[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) n[j] = g.nbr[3 * W.i + j];
+  ld4(a + W.s0, W.a);
+  ld4(b + W.s0, W.b);
+  load_col(g, W.i, W.C);
+  const uint32_t qq = (uint32_t)(W.k0 >> 2);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    W.d[j] = (uint32_t)n[j] * (uint32_t)g.NQ + qq - base;
+    if (W.d[j] >= W.lim) {
+      ld4(a + (size_t)n[j] * g.NS + W.k0, W.na[j]);
+      ld4(b + (size_t)n[j] * g.NS + W.k0, W.nb[j]);
+    }
+  }
+  if (W.k0 >= 1 && threadIdx.x == 0) {
+    W.am = a[W.s0 - 1];
+    W.bm = b[W.s0 - 1];
+  }
+  if (W.k0 + 4 <= g.NZ - 2 && threadIdx.x + 1 >= W.lim) {
+    W.ap = a[W.s0 + 4];
+    W.bp = b[W.s0 + 4];
+  }
+}
+
+// f = a + c b (a when first) at the seven points of the window's quads; body
+// as in for_each_quad_formed
+template <typename T, class Body>
+__device__ inline void win_apply(const Geo &g, Win<T> &W, T c, bool first, Body &&body) {
+  __shared__ __align__(16) T win[NSX_BLOCK][4];
+  T fc[4], fm = first ? W.am : W.am + c * W.bm, fp = first ? W.ap : W.ap + c * W.bp, fn[3][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) win[threadIdx.x][u] = fc[u] = first ? W.a[u] : W.a[u] + c * W.b[u];
+  __syncthreads();
+  if (!W.act) return;
+  if (W.k0 >= 1 && threadIdx.x >= 1) fm = win[threadIdx.x - 1][3];
+  if (W.k0 + 4 <= g.NZ - 2 && threadIdx.x + 1 < W.lim) fp = win[threadIdx.x + 1][0];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      fn[j][u] = W.d[j] < W.lim ? win[W.d[j]][u] : first ? W.na[j][u] : W.na[j][u] + c * W.nb[j][u];
+  body(fc, fm, fp, fn[0], fn[1], fn[2]);
+}
+
+__global__ __launch_bounds__(NSX_BLOCK) void k_bicg_a1(Geo g, const double *rt, const double *q, const double *rhat,
+                                                        double *vt, Partials P, SolverState *st) {
+  Win<double> W;
+  double tot[4], rh[4] = {0.0, 0.0, 0.0, 0.0}, qv[5];
+  const int done = st->done;
+  part_load<4>(P.c, tot);
+  win_load(g, rt, q, W);
+  if (W.act) ld4(rhat + W.s0, rh);
+  const double *lv = part_levels<4>(g, tot);
+  if (done) return;
+  double beta = 0.0;
+  bool first = false;
+  if (!begin_iteration(g, P, st, beta, first, st->c_iter == 0 ? nullptr : tot)) return;
+  if (W.act) quot5(W.C, lv, W.k0, qv);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->a_beta = beta;
+  double acc[1] = {0.0};
+  win_apply(g, W, beta, first, [&](const double(&yc)[4], double ym, double yp, const double(&y0)[4],
+                                   const double(&y1)[4], const double(&y2)[4]) {
+    double vo[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const Row1<double> R = row_of(g, lv, W.C, qv, W.k0, u);
+      const double v = apply_row(g, R, W.k0, u, yc, ym, yp, y0[u], y1[u], y2[u]);
+      vo[u] = R.in ? v / R.A0 : 0.0;
+      acc[0] += rh[u] * v;
+    }
+    st4(vt + W.s0, vo);
+  });
+  write_partials<1>(acc, P.a);
+}
+
+__global__ __launch_bounds__(NSX_BLOCK) void k_bicg_b1(Geo g, const double *rt, const double *vt, double *tv,
+                                                        Partials P, SolverState *st) {
+  Win<double> W;
+  double tr[1], qv[5];
+  const int done = st->done;
+  part_load<1>(P.a, tr);
+  win_load(g, rt, vt, W);
+  const double *lv = part_levels<1>(g, tr);
+  if (done) return;
+  if (W.act) quot5(W.C, lv, W.k0, qv);
+  const double al = st->a_rho[st->a_iter & 1] / tr[0];
+  if (fabs(tr[0]) < TINY || !isfinite(al)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      st->exit_code = EXIT_BREAKDOWN;
+      st->done = 1;
+    }
+    return;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->b_alpha = al;
+  double acc[2] = {0.0, 0.0};
+  win_apply(g, W, -al, false, [&](const double(&zc)[4], double zm, double zp, const double(&z0)[4],
+                                  const double(&z1)[4], const double(&z2)[4]) {
+    double t[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const Row1<double> R = row_of(g, lv, W.C, qv, W.k0, u);
+      t[u] = apply_row(g, R, W.k0, u, zc, zm, zp, z0[u], z1[u], z2[u]);
+      const double sd = R.in ? R.A0 * zc[u] : 0.0;
+      acc[0] += t[u] * sd;
+      acc[1] += t[u] * t[u];
+    }
+    st4(tv + W.s0, t);
+  });
+  write_partials<2>(acc, P.b);
 }
 
 // ------------------------------------------------ mixed-precision CG ----
@@ -1845,20 +2032,20 @@ int launch_bicg_init(const Geo &g, hipStream_t s, const double *rhs, const doubl
   return (int)hipGetLastError();
 }
 
-template <typename T>
-static int iter_impl(const Geo &g, hipStream_t s, T *x, T *rt, const T *rhat, T *q, T *vt, T *tv, Partials part,
-                     SolverState *st, hipEvent_t *ev) {
-  const dim3 grid(g.grid), blk(NSX_BLOCK);
-  const size_t lds = level_lds(g, sizeof(T));
-  LAUNCH_TIMED(ev, 0, k_bicg_a<T>, grid, blk, lds, s, g, (const T *)rt, (const T *)q, rhat, vt, part, st);
-  LAUNCH_TIMED(ev, 1, k_bicg_b<T>, grid, blk, lds, s, g, (const T *)rt, (const T *)vt, tv, part, st);
-  LAUNCH_TIMED(ev, 2, k_bicg_c<T>, grid, blk, lds, s, g, x, rt, q, rhat, (const T *)vt, (const T *)tv, part, st);
-  return (int)hipGetLastError();
-}
-
 int launch_bicg_iter(const Geo &g, hipStream_t s, double *x, double *rt, const double *rhat, double *q, double *vt,
                      double *tv, Partials part, SolverState *st, hipEvent_t *ev) {
-  return iter_impl<double>(g, s, x, rt, rhat, q, vt, tv, part, st, ev);
+  const dim3 grid(g.grid), blk(NSX_BLOCK);
+  const size_t lds = level_lds(g, sizeof(double));
+  const double *crt = rt, *cq = q, *cvt = vt, *ctv = tv;
+  if (g.one_window) {
+    LAUNCH_TIMED(ev, 0, k_bicg_a1, grid, blk, lds, s, g, crt, cq, rhat, vt, part, st);
+    LAUNCH_TIMED(ev, 1, k_bicg_b1, grid, blk, lds, s, g, crt, cvt, tv, part, st);
+  } else {
+    LAUNCH_TIMED(ev, 0, k_bicg_a<double>, grid, blk, lds, s, g, crt, cq, rhat, vt, part, st);
+    LAUNCH_TIMED(ev, 1, k_bicg_b<double>, grid, blk, lds, s, g, crt, cvt, tv, part, st);
+  }
+  LAUNCH_TIMED(ev, 2, k_bicg_c<double>, grid, blk, lds, s, g, x, rt, q, rhat, cvt, ctv, part, st);
+  return (int)hipGetLastError();
 }
 
 int launch_cg_init(const Geo &g, hipStream_t s, const double *rhs, const double *phi_in, double *x, float *rt,
@@ -1968,9 +2155,11 @@ int cg_blocks_per_cu(const Geo &g) {
   return n;
 }
 
-// resident blocks per CU of the single-reduction FP32 CG kernel
+// resident blocks per CU of the single-reduction FP32 CG kernel (point Jacobi
+// and blocks; the line instance holds more registers, and its last blocks
+// wait where the grid takes all of these)
 int cgs_blocks_per_cu(const Geo &g) {
-  const void *ks[3] = {(const void *)k_cgs<float, 0>, (const void *)k_cgs<float, 1>, (const void *)k_cgs<float, 2>};
+  const void *ks[2] = {(const void *)k_cgs<float, 0>, (const void *)k_cgs<float, 1>};
   int m = 1 << 30;
   for (const void *k : ks) {
     int n = 0;

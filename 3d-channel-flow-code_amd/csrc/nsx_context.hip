@@ -54,11 +54,15 @@ struct Xfer {
   double *pin[2] = {nullptr, nullptr}, *dev[2] = {nullptr, nullptr};
   hipEvent_t done[2] = {nullptr, nullptr};
   int nrow = 0, *src = nullptr;  // the ghost rows filled and their device columns
-  std::vector<int> row;
+  std::vector<int> row, hsrc;    // (their host rows, the columns again)
   bool contiguous = false;       // every ghost row, in order
 };
 // 4 MB: a chunk's crossing (70 us) hides its launches, two stay in the host's cache
 #define NSX_XFER_CHUNK (512 * 1024)
+// up to so many values the host transposes (a kernel's launch costs more: at 6,528
+// values a stage's 18 transfers took 100 us longer with it; at 36,864 it saves 30 %
+// of the single routines' calls)
+#define NSX_XFER_HOST 16384
 
 struct nsx_ctx {
   int N0 = 0, NC = 0, NV = 0, NZ = 0, NS = 0, NEX = 0;
@@ -406,42 +410,37 @@ extern "C" int nsx_commit(nsx_ctx *ctx) {
     HIPCHECK(hipGetDeviceProperties(&prop, ctx->dev));
     const int per_cu = solver_blocks_per_cu(g);
     if (per_cu < 1) return nsx_fail(ctx, -2, "occupancy query of the solver kernels failed");
-    long G = (long)prop.multiProcessorCount * per_cu;
     const long need = ((long)g.nquad + NSX_BLOCK - 1) / NSX_BLOCK;
-    if (G > need) G = need;
-    if (G > MAXGRID) G = MAXGRID;
-    G = G / NSX_NXCD * NSX_NXCD;
-    if (G < NSX_NXCD) G = NSX_NXCD;
-    g.grid = (int)G;
+    // every block resident at once, a whole number per XCD (rounded up where
+    // the windows are fewer: rounded down, 36 windows ran as two rounds on
+    // 32 blocks)
+    auto grid_of = [&](int per) {
+      long G = (long)prop.multiProcessorCount * per;
+      if (G > MAXGRID) G = MAXGRID;
+      G = G / NSX_NXCD * NSX_NXCD;
+      if (G > need) G = (need + NSX_NXCD - 1) / NSX_NXCD * NSX_NXCD;
+      return (int)(G < NSX_NXCD ? NSX_NXCD : G);
+    };
+    g.grid = grid_of(per_cu);
+    g.one_window = need <= NSX_ONE_WINDOW;
+    if (g.one_window) g.grid = (int)need;
     const int per_cu_cg = cg_blocks_per_cu(g);
     if (per_cu_cg < 1) return nsx_fail(ctx, -2, "occupancy query of the CG kernels failed");
-    long Gc = (long)prop.multiProcessorCount * per_cu_cg;
-    if (Gc > need) Gc = need;
-    if (Gc > MAXGRID) Gc = MAXGRID;
-    Gc = Gc / NSX_NXCD * NSX_NXCD;
-    if (Gc < NSX_NXCD) Gc = NSX_NXCD;
-    g.grid_cg = (int)Gc;
+    g.grid_cg = grid_of(per_cu_cg);
     // the single-reduction CG kernel runs 4 blocks a CU, below its occupancy
     // (5): at 6.3M prisms 1024 blocks sweep 6 windows each, a band per XCD
     // that its L2 holds, and took 50.5 us a launch against 52.2 us for 1280
     // (896: 52.5, 1152: 51.8)
-    const int per_cu_cgs = std::min(cgs_blocks_per_cu(g), 4);
+    // ... and one round where its occupancy allows that: at 1,088 windows 1,024
+    // blocks took a second round for 64 of them
+    const int occ_cgs = cgs_blocks_per_cu(g);
+    const int per_cu_cgs = need <= (long)prop.multiProcessorCount * occ_cgs ? occ_cgs : std::min(occ_cgs, 4);
     if (per_cu_cgs < 1) return nsx_fail(ctx, -2, "occupancy query of the single-reduction CG kernel failed");
-    long Gs = (long)prop.multiProcessorCount * per_cu_cgs;
-    if (Gs > need) Gs = need;
-    if (Gs > MAXGRID) Gs = MAXGRID;
-    Gs = Gs / NSX_NXCD * NSX_NXCD;
-    if (Gs < NSX_NXCD) Gs = NSX_NXCD;
-    g.grid_cgs = (int)Gs;
+    g.grid_cgs = grid_of(per_cu_cgs);
     // its FP64 instance: every block its occupancy allows, at most 4 a CU
     const int per_cu_64 = std::min(cgs64_blocks_per_cu(g), 4);
     if (per_cu_64 < 1) return nsx_fail(ctx, -2, "occupancy query of the FP64 single-reduction CG kernel failed");
-    long G6 = (long)prop.multiProcessorCount * per_cu_64;
-    if (G6 > need) G6 = need;
-    if (G6 > MAXGRID) G6 = MAXGRID;
-    G6 = G6 / NSX_NXCD * NSX_NXCD;
-    if (G6 < NSX_NXCD) G6 = NSX_NXCD;
-    g.grid_cgs64 = (int)G6;
+    g.grid_cgs64 = grid_of(per_cu_64);
   }
   if (NS > 4096) return nsx_fail(ctx, -1, "NZ = %d exceeds the 4094 layers the solver's LDS level table holds", NZ);
   g.bctop = ctx->bctop;
@@ -834,6 +833,7 @@ static int xfer_setup(nsx_ctx *ctx) {
   }
   X.nrow = (int)src.size();
   X.contiguous = X.nrow == ctx->NEX - N0;
+  X.hsrc = src;
   int rc;
   if ((rc = dev_upload(ctx, &X.src, src))) return rc;
   // a chunk holds at least one layer of every kind of field
@@ -862,6 +862,16 @@ extern "C" int nsx_put_field(nsx_ctx *ctx, int f, const double *host) {
   const int ngw = kind == FK_CELL ? ctx->NGW : 0, n = vert ? ctx->NV : N0, w = n + ngw;
   const size_t ld = vert ? (size_t)ctx->NV : kind == FK_FACE ? (size_t)N0 : (size_t)ctx->NC;
   const int kz = vert ? ctx->NZ - 1 : ctx->NZ, stride = vert ? ctx->NZ - 1 : ctx->NS;
+  const size_t ne = field_elems(ctx, kind);
+  if (ne <= NSX_XFER_HOST) {
+    for (int c = 0; c < w; ++c)
+      for (int k = 0; k < stride; ++k)
+        X.pin[0][(size_t)c * stride + k] =
+            k < kz ? host[(size_t)(c < n ? c : ctx->gw_ghost[c - n]) + (size_t)k * ld] : 0.0;
+    HIPCHECK(hipMemcpyAsync(ctx->slot[f], X.pin[0], ne * sizeof(double), hipMemcpyHostToDevice, s));
+    HIPCHECK(hipStreamSynchronize(s));
+    return 0;
+  }
   const int step = std::max(1, (int)(X.chunk / (size_t)w));
   for (int k0 = 0, c = 0; k0 < stride; k0 += step, ++c) {
     const int nk = std::min(step, stride - k0), q = c & 1;
@@ -897,6 +907,17 @@ extern "C" int nsx_get_field(nsx_ctx *ctx, int f, double *host, int fill_ghost_r
   const int n = vert ? ctx->NV : N0, w = n + (ghosts ? X.nrow : 0);
   const size_t ld = vert ? (size_t)ctx->NV : kind == FK_FACE ? (size_t)N0 : (size_t)ctx->NC;
   const int kz = vert ? ctx->NZ - 1 : ctx->NZ, stride = vert ? ctx->NZ - 1 : ctx->NS;
+  const size_t ne = field_elems(ctx, kind);
+  if (ne <= NSX_XFER_HOST) {
+    HIPCHECK(hipMemcpyAsync(X.pin[0], ctx->slot[f], ne * sizeof(double), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipStreamSynchronize(s));
+    for (int k = 0; k < kz; ++k) {
+      double *dst = host + (size_t)k * ld;
+      for (int c = 0; c < n; ++c) dst[c] = X.pin[0][(size_t)c * stride + k];
+      for (int e = 0; e < w - n; ++e) dst[X.row[e]] = X.pin[0][(size_t)X.hsrc[e] * stride + k];
+    }
+    return 0;
+  }
   const int step = std::max(1, (int)(X.chunk / (size_t)w)), nchunk = (kz + step - 1) / step;
   auto issue = [&](int c) -> int {
     const int k0 = c * step, nk = std::min(step, kz - k0), q = c & 1;

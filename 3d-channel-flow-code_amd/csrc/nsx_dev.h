@@ -59,6 +59,7 @@ struct Geo {
   uint32_t ncell;           // N0*NZi interior prisms
   int NQ;                   // NS/4 four-layer groups per column
   int grid;                 // grid of the kernels that produce or consume solver partial sums
+  int one_window;           // 1: the BiCGSTAB phases work on one window a block (grid = windows)
   int grid_cg;              // grid of the FP32 CG stencil kernel (its own occupancy)
   int grid_cgs;             // grid of the single-reduction FP32 CG kernel (its own occupancy)
   int grid_cgs64;           // grid of its FP64 instance

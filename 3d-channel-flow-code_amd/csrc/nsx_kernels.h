@@ -16,6 +16,10 @@
       hipLaunchKernelGGL(kern, grid, blk, lds, s, __VA_ARGS__);                                 \
   } while (0)
 
+// the most windows of NSX_BLOCK quads on which the BiCGSTAB phases take one
+// window a block
+#define NSX_ONE_WINDOW 512
+
 // Per-block partial sums of one reduction site: [rows][grid]
 struct Partials {
   double *src;   // Glob_Norm(rhs,1) sum (k_source / k_gnorm_sum), 1 row

@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nx, ny, nn, walls", [
-    (2, 2, 2, None),          # one tile, one chunk
+    (2, 2, 2, None),          # small enough for the host to transpose
+    (21, 11, 29, (1, 0, 0, 0)),  # the same with walls
+    (32, 8, 30, None),        # 16,384 values: the most of those
     (33, 17, 31, (1, 0, 0, 0)),  # odd columns and layers, wall ghost rows
     (32, 16, 30, None),       # as many layers as a tile
     (90, 45, 67, None),       # 4.5 MB: two chunks, the last ragged
