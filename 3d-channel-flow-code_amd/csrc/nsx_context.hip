@@ -7,6 +7,9 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <atomic>
+#include <exception>
+#include <thread>
 #include <vector>
 
 #include "nsx.h"
@@ -63,6 +66,8 @@ struct Xfer {
 // values a stage's 18 transfers took 100 us longer with it; at 36,864 it saves 30 %
 // of the single routines' calls)
 #define NSX_XFER_HOST 16384
+// values from which four threads copy (16 MB)
+#define NSX_XFER_THREADS (2 * 1024 * 1024)
 
 struct nsx_ctx {
   int N0 = 0, NC = 0, NV = 0, NZ = 0, NS = 0, NEX = 0;
@@ -431,10 +436,9 @@ extern "C" int nsx_commit(nsx_ctx *ctx) {
     // (5): at 6.3M prisms 1024 blocks sweep 6 windows each, a band per XCD
     // that its L2 holds, and took 50.5 us a launch against 52.2 us for 1280
     // (896: 52.5, 1152: 51.8)
-    // ... and one round where its occupancy allows that: at 1,088 windows 1,024
-    // blocks took a second round for 64 of them
-    const int occ_cgs = cgs_blocks_per_cu(g);
-    const int per_cu_cgs = need <= (long)prop.multiProcessorCount * occ_cgs ? occ_cgs : std::min(occ_cgs, 4);
+    // (also where 1,088 windows would be one round of 1,088 blocks: 18.0 us a
+    // launch on 1,024, 19.5 on 1,088)
+    const int per_cu_cgs = std::min(cgs_blocks_per_cu(g), 4);
     if (per_cu_cgs < 1) return nsx_fail(ctx, -2, "occupancy query of the single-reduction CG kernel failed");
     g.grid_cgs = grid_of(per_cu_cgs);
     // its FP64 instance: every block its occupancy allows, at most 4 a CU
@@ -928,6 +932,50 @@ extern "C" int nsx_get_field(nsx_ctx *ctx, int f, double *host, int fill_ghost_r
     HIPCHECK(hipEventRecord(X.done[q], s));
     return 0;
   };
+  // rows that no rule fills stay as the caller left them
+  const bool whole = w == n || X.contiguous;
+  auto copy_rows = [&](int c, int first, int every) {
+    const int k0 = c * step, nk = std::min(step, kz - k0);
+    for (int k = first; k < nk; k += every) {
+      const double *src = X.pin[c & 1] + (size_t)k * w;
+      double *dst = host + (size_t)(k0 + k) * ld;
+      memcpy(dst, src, (size_t)(whole ? w : n) * sizeof(double));
+      if (!whole)
+        for (int e = 0; e < X.nrow; ++e) dst[X.row[e]] = src[n + e];
+    }
+  };
+  // The crossing waits for the host's copy (and the page faults of a fresh
+  // array): large fields are copied by four threads, each taking every fourth
+  // layer of a chunk.  `ready` counts the chunks that have arrived (or -1: an
+  // error ended the call), `copied` the shares done.
+  const int nt = step >= 4 && (size_t)kz * w >= NSX_XFER_THREADS ? 4 : 1;
+  std::atomic<int> ready{0}, copied{0};
+  std::vector<std::thread> team;
+  struct Join {
+    std::atomic<int> &ready;
+    std::vector<std::thread> &team;
+    ~Join() {
+      if (!team.empty()) ready.store(-1);
+      for (std::thread &t : team) t.join();
+    }
+  };
+  const Join join{ready, team};
+  auto work = [&](int me) {
+    for (int c = 0; c < nchunk; ++c) {
+      int r;
+      while ((r = ready.load()) >= 0 && r <= c) std::this_thread::yield();
+      if (r < 0) return;
+      copy_rows(c, me, nt);
+      copied.fetch_add(1);
+    }
+  };
+  int helpers = 0;
+  try {
+    team.reserve(nt);
+    for (int q = 1; q < nt; ++q, ++helpers) team.emplace_back(work, q);
+  } catch (const std::exception &) {
+    // no more threads to be had: the shares without one are this thread's
+  }
   if ((rc = issue(0))) return rc;
   for (int c = 0; c < nchunk; ++c) {
     if (c + 1 < nchunk && (rc = issue(c + 1))) return rc;
@@ -935,16 +983,11 @@ extern "C" int nsx_get_field(nsx_ctx *ctx, int f, double *host, int fill_ghost_r
       HIPCHECK(hipStreamSynchronize(s));
     else
       HIPCHECK(hipEventSynchronize(X.done[c & 1]));
-    const int k0 = c * step, nk = std::min(step, kz - k0);
-    for (int k = 0; k < nk; ++k) {
-      const double *src = X.pin[c & 1] + (size_t)k * w;
-      double *dst = host + (size_t)(k0 + k) * ld;
-      // rows that no rule fills stay as the caller left them
-      const bool whole = w == n || X.contiguous;
-      memcpy(dst, src, (size_t)(whole ? w : n) * sizeof(double));
-      if (!whole)
-        for (int e = 0; e < X.nrow; ++e) dst[X.row[e]] = src[n + e];
-    }
+    ready.store(c + 1);
+    copy_rows(c, 0, nt);
+    for (int q = helpers + 1; q < nt; ++q) copy_rows(c, q, nt);
+    // the next transfer into this chunk's buffer is issued after this
+    while (copied.load() < helpers * (c + 1)) std::this_thread::yield();
   }
   return 0;
 }

@@ -192,7 +192,11 @@ static int launch_transform(const Geo &g, hipStream_t s, const ModalDev &M, cons
 // before and after the coarse correction, a degree-2 Chebyshev polynomial on
 // [lmax / 4, lmax] on the levels below (lmax: Gershgorin's bound of the
 // mode's D^-1 A), a dense inverse on the coarsest.  The block's only
-// synchronisation is its own barrier.
+// synchronisation is its own barrier.  4,096 columns x 48 modes: 0.5 ms for 20
+// to 25 iterations, bound by latency (24 cycles a vector memory instruction,
+// the vector units 21 % busy).  Four nodes' loads ahead, reciprocals kept
+// instead of divisions, and the columns' state in registers gained nothing (the
+// last spills).
 constexpr int T2 = 1024;  // threads of a 2D block
 constexpr int W2 = T2 / 64;
 

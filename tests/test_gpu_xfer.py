@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (32, 16, 30, None),       # as many layers as a tile
     (90, 45, 67, None),       # 4.5 MB: two chunks, the last ragged
     (128, 64, 64, (0, 0, 0, 0)),  # three chunks
+    (180, 91, 67, None),      # 18 MB: several threads copy
 ])
 def test_round_trip(nx, ny, nn, walls):
     from nsx.device import Context
