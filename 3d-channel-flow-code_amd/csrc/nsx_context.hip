@@ -1265,9 +1265,10 @@ static int modal_setup(nsx_ctx *ctx) {
   M.mp = 16 * M.kt;
   M.batched = N0 >= NSX_MODAL_BATCH && M.nlev >= 3 && M.mp <= 4 * NSX_BLOCK;
   // the transforms' panels: the most output tiles whose part of the table
-  // fits the LDS (and the accumulators eight), spread evenly
-  const int tile = M.kt * 256 * (int)sizeof(double), most = std::min(8, lds / tile);
-  if (most < 1) return nsx_fail(ctx, -1, "vertical-mode solve: %d layers pass the mode table's LDS", nzi);
+  // fits the LDS beside the partial sums' (and the accumulators eight), spread
+  // evenly; where not one fits, a tile a panel, read from global memory
+  const int tile = M.kt * 256 * (int)sizeof(double), fits = std::min(8, (lds - 256) / tile);
+  const int most = std::max(1, fits);
   M.npanel = (M.kt + most - 1) / most;
   M.mt = (M.kt + M.npanel - 1) / M.npanel;
   {
@@ -1275,10 +1276,11 @@ static int modal_setup(nsx_ctx *ctx) {
     const int per = std::max(1, std::min(4, lds / (M.mt * tile))), want = (M.N0p / 16 + 3) / 4;
     M.agrid = std::max(1, std::min(want, std::max(1, per * prop.multiProcessorCount / M.npanel)));
   }
-  const int MP = 16 * M.kt, ntab = M.npanel * M.mt * M.kt * 256;
+  const int MP = 16 * M.kt, ntab = M.npanel * M.mt * M.kt * 256, nout = M.npanel * M.mt;
+  if (fits < 1) M.mt = 0;
   auto phik = [&](int k, int m) -> double { return (k < nzi && m < nzi) ? H.phi[(size_t)k * nzi + m] : 0.0; };
   std::vector<double> tf((size_t)ntab, 0.0), tb((size_t)ntab, 0.0), mu((size_t)MP, 1.0);
-  for (int o = 0; o < M.npanel * M.mt; ++o)
+  for (int o = 0; o < nout; ++o)
     for (int t = 0; t < M.kt; ++t)
       for (int lane = 0; lane < 64; ++lane)
         for (int q = 0; q < 4; ++q) {

@@ -110,7 +110,7 @@ struct ModalDev {
   int nzi, nlev, nc;
   int N0, N0p;  // columns, and padded to a multiple of 16 (the row length of bh, xh)
   int kt;       // 16-wide tiles of layers (and of modes)
-  int mt;       // output tiles a transform block forms (a panel), and the panels
+  int mt;       // output tiles a transform block forms (a panel; 0: one, from global memory), and the panels
   int npanel;
   int agrid;    // blocks of the transform kernels along the columns
   int lds2d;    // dynamic LDS of the 2D solve, bytes

@@ -22,11 +22,14 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 // table's operands are laid out by the host so that a lane's four are one
 // 32-byte run in LDS; a block holds the table's panel of MT output tiles (at
 // 96 layers all six, 72 KB: two blocks a CU; npanel > 1 where the whole table
-// passes the LDS).
+// passes the LDS).  MT = 0: one output tile a block whose operands come from
+// global memory, for tables of which not one tile fits (more than 1,264
+// layers); the LDS form stays the one wherever it fits.
 constexpr int MODAL_TB = 256;
 
 template <int MT>
 __device__ inline const double *lds_panel(const double *src, int kt) {
+  if constexpr (MT == 0) return src;
   extern __shared__ __align__(16) unsigned char nsx_dyn_lds[];
   double2 *dst = reinterpret_cast<double2 *>(nsx_dyn_lds);
   const double2 *s = reinterpret_cast<const double2 *>(src);
@@ -50,8 +53,9 @@ __device__ inline void load_layers(const double *p, int k, int nzi, bool ok, dou
 template <int MT, bool NODE>
 __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const double *r, const SolverState *st) {
   if (st->done) return;
-  const int kt = M.kt, nzi = M.nzi, m0 = 16 * MT * (int)blockIdx.y;
-  const double *tab = lds_panel<MT>(M.tfwd + (size_t)blockIdx.y * MT * kt * 256, kt);
+  constexpr int NT = MT ? MT : 1;
+  const int kt = M.kt, nzi = M.nzi, m0 = 16 * NT * (int)blockIdx.y;
+  const double *tab = lds_panel<MT>(M.tfwd + (size_t)blockIdx.y * NT * kt * 256, kt);
   const int lane = threadIdx.x & 63, j = lane & 15, gq = lane >> 4;
   const int ntile = M.N0p >> 4, stride = gridDim.x * (MODAL_TB / 64);
   double sum[1] = {0.0};
@@ -59,9 +63,9 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
     const int c = 16 * tile + j;
     const bool ok = c < g.N0;
     const double *src = r + (size_t)(ok ? c : 0) * g.NS + 1;
-    f64x4 acc[MT];
+    f64x4 acc[NT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int m = 0; m < NT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
     double b[4], bn[4];
     load_layers(src, 4 * gq, nzi, ok, b);
     for (int t = 0; t < kt; ++t) {
@@ -70,7 +74,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+        for (int m = 0; m < NT; ++m)
           acc[m] = NODE ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[q], a[(size_t)m * kt * 256 + q], acc[m], 0, 0, 0)
                         : __builtin_amdgcn_mfma_f64_16x16x4f64(a[(size_t)m * kt * 256 + q], b[q], acc[m], 0, 0, 0);
 #pragma unroll
@@ -82,7 +86,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
       for (int q = 0; q < 4; ++q) {
         double *dst = M.bh + (size_t)(16 * tile + gq + 4 * q) * M.mp + m0 + j;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
+        for (int m = 0; m < NT; ++m) {
           if (m0 + 16 * m < M.mp) dst[16 * m] = acc[m][q];
           sum[0] += acc[m][q] * acc[m][q];
         }
@@ -91,7 +95,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
     }
     // lanes j: 16 consecutive columns of one mode, a 128-byte run
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < NT; ++m)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int mode = m0 + 16 * m + gq + 4 * q;
@@ -106,19 +110,20 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_fwd(Geo g, ModalDev M, const
 template <int MT, bool NODE>
 __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, double *x, SolverState *st) {
   if (st->done) return;
+  constexpr int NT = MT ? MT : 1;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
     st->m_iters += st->m_cyc;
     st->m_cyc = 0;
     st->mp_pass += 1;
   }
-  const int kt = M.kt, nzi = M.nzi, l0 = 16 * MT * (int)blockIdx.y;
-  const double *tab = lds_panel<MT>(M.tbwd + (size_t)blockIdx.y * MT * kt * 256, kt);
+  const int kt = M.kt, nzi = M.nzi, l0 = 16 * NT * (int)blockIdx.y;
+  const double *tab = lds_panel<MT>(M.tbwd + (size_t)blockIdx.y * NT * kt * 256, kt);
   const int lane = threadIdx.x & 63, j = lane & 15, gq = lane >> 4;
   const int ntile = M.N0p >> 4, stride = gridDim.x * (MODAL_TB / 64);
   for (int tile = blockIdx.x * (MODAL_TB / 64) + (threadIdx.x >> 6); tile < ntile; tile += stride) {
-    f64x4 acc[MT];
+    f64x4 acc[NT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int m = 0; m < NT; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
     // xh's padding modes and columns are zero
     const double *src = NODE ? M.xh + (size_t)(16 * tile + j) * M.mp + 4 * gq
                              : M.xh + (size_t)(4 * gq) * M.N0p + 16 * tile + j;
@@ -134,7 +139,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, doubl
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+        for (int m = 0; m < NT; ++m)
           acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[(size_t)m * kt * 256 + q], acc[m], 0, 0, 0);
 #pragma unroll
       for (int q = 0; q < 4; ++q) a[q] = an[q];
@@ -146,7 +151,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, doubl
       if (c >= g.N0) continue;
       double *dst = x + (size_t)c * g.NS + 1;
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
+      for (int m = 0; m < NT; ++m) {
         const int k = l0 + 16 * m + j;
         if (k < nzi) dst[k] -= acc[m][q];
       }
@@ -173,6 +178,7 @@ static int launch_transform_t(const Geo &g, hipStream_t s, const ModalDev &M, co
 static int launch_transform(const Geo &g, hipStream_t s, const ModalDev &M, const double *r, double *x,
                             SolverState *st, bool fwd, hipEvent_t *ev) {
   switch (M.mt) {
+    case 0: return launch_transform_t<0>(g, s, M, r, x, st, fwd, ev);
     case 1: return launch_transform_t<1>(g, s, M, r, x, st, fwd, ev);
     case 2: return launch_transform_t<2>(g, s, M, r, x, st, fwd, ev);
     case 3: return launch_transform_t<3>(g, s, M, r, x, st, fwd, ev);
@@ -497,7 +503,7 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
 // Levels 2 and below run one block per mode in LDS.  Modes whose residual has
 // met its target stop; the rows are swept up to the last mode still
 // iterating.  At 6.3M prisms with all modes iterating the update moves 350 MB
-// in 75 us (4.6 TB/s) and the product 126 MB and its gathers in 46 us; with few modes the 20
+// in 75 us (4.6 TB/s) and the product 126 MB and its gathers in 46 us; with few modes the 18
 // launches' latency bounds the iteration.
 constexpr int MB = NSX_BLOCK;
 
@@ -986,6 +992,7 @@ bool modal_allow_lds(const ModalDev &M) {
   const bool ok = M.batched ? allow(reinterpret_cast<const void *>(&k_mb_below), M.lds2d)
                             : allow(reinterpret_cast<const void *>(&k_modal_2d), M.lds2d);
   switch (M.mt) {
+    case 0: return ok;
     case 1: return ok && allow_t<1>(tr);
     case 2: return ok && allow_t<2>(tr);
     case 3: return ok && allow_t<3>(tr);

@@ -83,3 +83,27 @@ def test_modal_zero_and_solved_right_hand_sides():
     G.close()
     assert info["exit"] == "no solve" and info["iters"] == 0, info
     assert rel_err(interior(c, again), interior(c, phi)) <= 1e-12
+
+
+@pytest.mark.parametrize("nn", [
+    320,     # twenty tiles: four tiles' operands are the whole LDS
+    1265,    # eighty tiles: one tile's operands are
+    1300,    # not one tile's fit
+])
+def test_modal_deep_columns(nn):
+    """The residual alone is checked: at these depths the operator's condition
+    number, about the layers squared, leaves the pressures of two solves fewer
+    common digits."""
+    from nsx.device import Context
+    c = make_case(3, 2, nn, seed=4, jitter=0.1)
+    rhs = c.cell_field()
+    rhs[:c.N_CELL0, 1:-1] = np.random.default_rng(nn).standard_normal((c.N_CELL0, c.NZ - 2))
+    G = Context(c)
+    G.set_params(eps=1e-8)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    G.init_state()
+    phi, _, info = G.bicgstab(c.cell_field(), rhs)
+    G.close()
+    assert info["exit"] == "converged" and info["iters_fp32"] == info["iters"] > 0, info
+    e1, e2 = ppe_residual(c, phi, rhs)
+    assert min(e1, e2) < 2e-8, (e1, e2)
