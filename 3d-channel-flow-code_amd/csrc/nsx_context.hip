@@ -141,7 +141,7 @@ struct nsx_ctx {
   ModalDev modal{};
   bool modal_ok = false;
   Xfer xfer;
-  int modal_cycles = 0, modal_iters = 44;
+  int modal_cycles = 2, modal_iters = 44, modal_more = 12;
   int iter_hint_cg = 0;
   int iter_hint_cgs = 0;
   int iter_hint_cgs64 = 0;
@@ -1412,7 +1412,7 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
   LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 1, cap));
   const size_t pend0 = ctx->pending.size();
   // as many cycles as the last solve took, then one at a time
-  for (int cycles = std::max(1, ctx->modal_cycles), issued = 0;; cycles = 1) {
+  for (int cycles = std::max(2, ctx->modal_cycles), issued = 0;; cycles = 1) {
     for (int c = 0; c < cycles; ++c, ++issued) {
       hipEvent_t *ev = nullptr;
       if (ctx->timing) {
@@ -1420,7 +1420,8 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
         if (!ev) return nsx_fail(ctx, -2, "hipEventCreate failed");
       }
       LAUNCH(launch_modal_fwd(g, s, ctx->modal, r, ctx->st_dev, ev));
-      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, ctx->modal_iters, ev ? ev + 2 : nullptr));
+      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, issued ? ctx->modal_more : ctx->modal_iters,
+                             ev ? ev + 2 : nullptr));
       LAUNCH(launch_modal_bwd(g, s, ctx->modal, x, ctx->st_dev, ev ? ev + 4 : nullptr));
       LAUNCH(launch_modal_true(g, s, rhs, x, r, ctx->part, ctx->st_dev, ev ? ev + 6 : nullptr));
       LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 0, cap));
@@ -1441,8 +1442,9 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
   const int it = h.m_iters;
   if (h.mp_pass > 0) {
     ctx->modal_cycles = h.mp_pass;
-    // the iterations the whole solve took, a few more: one cycle should do
-    ctx->modal_iters = std::min(NSX_MB_ITERS, std::max(8, it + 4));
+    // the iterations the first cycle took and those after it, a few more
+    ctx->modal_iters = std::min(NSX_MB_ITERS, std::max(8, h.m_first + 4));
+    if (h.mp_pass > 1) ctx->modal_more = std::min(NSX_MB_ITERS, std::max(6, (it - h.m_first) / (h.mp_pass - 1) + 4));
   }
   if (h.exit_code == NSX_SOLVE_MAX_ITERS || h.exit_code == NSX_SOLVE_BREAKDOWN)
     return finish_fp64(ctx, rhs, x, it, h.mp_pass);

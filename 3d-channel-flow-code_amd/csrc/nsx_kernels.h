@@ -80,7 +80,7 @@ struct SolverState {
   int m_stall;        // cycles in a row that did not lower it by a tenth        (check kernel)
   int m_cyc;          // most iterations of a mode in this cycle                 (2D solves; backward transform: 0)
   int m_iters;        // sum of m_cyc over the cycles                            (backward transform)
-  int pad4;
+  int m_first;        // m_cyc of the first cycle                                  (backward transform)
 };
 
 // the vectors of the single-reduction CG: e and p in place, the scaled

@@ -112,6 +112,7 @@ __global__ __launch_bounds__(MODAL_TB) void k_modal_bwd(Geo g, ModalDev M, doubl
   if (st->done) return;
   constexpr int NT = MT ? MT : 1;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    if (st->mp_pass == 0) st->m_first = st->m_cyc;
     st->m_iters += st->m_cyc;
     st->m_cyc = 0;
     st->mp_pass += 1;
