@@ -1,6 +1,6 @@
 """The FP64 BiCGSTAB either side of the sizes where its launches change shape:
 one window of 256 quads and less, a last window of one quad, as many windows as
-take one a block (512) and one more row of columns.  A random right-hand side
+take one a block (160) and one more, 512 and one more row of columns.  A random right-hand side
 solved to 1e-12: the host-checked residual meets the reference's rule (2 eps
 for the summation order), the pressure agrees with the vertical-mode solve's
 (eps times the operator's condition number, below 1e5 here: 1e-7), and a
@@ -22,6 +22,8 @@ EPS = 1e-12
     (16, 8, 2, None),          # 256: one window
     (43, 3, 2, (1, 0, 0, 0)),  # 258: two quads in the second
     (32, 16, 32, None),        # 36 windows, not a multiple of the XCDs
+    (80, 85, 10, None),        # 160 windows: the most one window a block takes
+    (72, 95, 10, None),        # 161: the general form
     (176, 124, 10, None),      # 512 windows
     (190, 115, 10, None),      # 513
 ])
