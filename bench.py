@@ -13,12 +13,11 @@ rule min(|r|_1/|b|_1, |r|_2/|b|_2) < eps):
   fp64_cg  single-reduction CG with the 4-layer block-Jacobi
            preconditioner in FP64 (separates the gain of a CG solver from
            the gain of FP32);
-  mixed    the precision form: FP32 CG preconditioned by the vertical modes
-           of the operator (NSX_REFINE_MODAL: per column the generalized
+  mixed    the precision form: the solve by the vertical modes of the
+           operator (NSX_REFINE_MODAL: per column the generalized
            eigenvectors of the vertical couplings split the PPE into one 2D
-           problem per mode; the 16 lowest by a V-cycle of aggregation
-           multigrid, the others by their diagonal), in cycles restarted
-           from the true FP64 residual, stopped on it;
+           problem per mode, each solved by FP64 CG with an FP32
+           multigrid), in cycles from the true FP64 residual, stopped on it;
   mixed_block  the previous precision form: the single-reduction block-
            Jacobi CG of fp64_cg in FP32 with reliable updates;
   mixed_flux32  the mixed leg with the momentum fluxes and the Smagorinsky
@@ -118,9 +117,8 @@ def cpu_baseline(case, mean_iters: float, cap: int = 100, parallel: bool = False
             "s_per_step": step_s}
 
 
-# the mixed forms (refinement, reliable-update delta): "mixed" the FP32 CG
-# with the vertical-mode preconditioner (delta unused: its cycles end on the
-# drop of rho); "mixed_block" the single-reduction FP32 CG with the 4-layer
+# the mixed forms (refinement, reliable-update delta): "mixed" the vertical-mode
+# solve (delta unused); "mixed_block" the single-reduction FP32 CG with the 4-layer
 # block-Jacobi preconditioner (the library's default), "mixed_line" the same
 # with the line preconditioner (whole columns), "mixed_point" with point
 # Jacobi; "mixed_cg2" the point-Jacobi CG in two kernels per iteration
@@ -150,7 +148,9 @@ def modal_kernels(case) -> dict:
     most = max(1, min(8, 160 * 1024 // (kt * 2048)))
     panels = (kt + most - 1) // most
     mt = (kt + panels - 1) // panels
-    return {"modal_fwd": ("k_modal_fwd<%d>" % mt, 16 * n), "modal_bwd": ("k_modal_bwd<%d>" % mt, 24 * n),
+    # node-major modal vectors where the 2D solves run batched
+    kind = "<%d, %s>" % (mt, "true" if case.N_CELL0 >= 24576 else "false")
+    return {"modal_fwd": ("k_modal_fwd" + kind, 16 * n), "modal_bwd": ("k_modal_bwd" + kind, 24 * n),
             "modal_spmv": ("k_modal_true", 24 * n), "modal_mg": ("2D solves of every mode", 0)}
 
 
@@ -329,14 +329,14 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": ("f32+f64 (vertical-mode-preconditioned FP32 CG, MFMA FP32 transforms, FP64 true residuals)"
+        "dtype": ("f64+f32 (FP64 CG per vertical mode, FP32 multigrid, MFMA FP64 transforms, FP64 true residuals)"
                   if "mixed" in res else ("f64" if "fp64" in res else "f32+f64")),
         "data": "synthetic",
         "config": {"workload": f"channel {WORKLOAD[cfg]}", "prisms": case.n_interior,
                    "time_scheme": "RK2 (FinRK=2)", "les": "Smagorinsky Cs=0.1", "ppe_tolerance": args.eps_gate,
                    "ppe_tolerance_workload": case.params.eps,
-                   "ppe_solver": "FP32 CG, vertical-mode preconditioner (16 modes by 2D aggregation multigrid), "
-                                 "cycles restarted from FP64 true residuals",
+                   "ppe_solver": "vertical-mode solve: FP64 CG per mode with an FP32 smoothed-aggregation V-cycle, "
+                                 "cycles from FP64 true residuals",
                    "initial_guess": {"precision_forms": args.guess, "fp64": "previous"},
                    "seed": args.seed},
         "roofline": {"bound": "hbm", "kernel": dom["kernel"], "achieved": dom["GBps"], "peak": HBM_PEAK_GBS,
