@@ -643,7 +643,14 @@ __global__ __launch_bounds__(T2) void k_mb_scalars(ModalDev M, SolverState *st, 
   } else {
     S.rr = s;
     S.act = S.act && s > S.target;
-    if (S.act) atomicMax(&M.nact[it + 1], m + 1);
+    if (S.act) {
+      atomicMax(&M.nact[it + 1], m + 1);
+    } else {
+      // the sweeps go on over its group of four, and these scalars are not
+      // formed again past the last mode still iterating: no further step
+      S.as = 0.0;
+      S.beta = 0.f;
+    }
     if (m == 0) st->m_cyc = it + 1;
   }
 }

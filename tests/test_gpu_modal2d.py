@@ -107,3 +107,47 @@ def test_modal_deep_columns(nn):
     assert info["exit"] == "converged" and info["iters_fp32"] == info["iters"] > 0, info
     e1, e2 = ppe_residual(c, phi, rhs)
     assert min(e1, e2) < 2e-8, (e1, e2)
+
+
+def _modes(c):
+    """the vertical modes, columns of (NZ-2) x (NZ-2), and the layers' S"""
+    n = c.NZ - 2
+    t, S = 1.0 / c.dsig[1:n], c.dsigv[:n]
+    T = np.zeros((n, n))
+    for q in range(n - 1):
+        T[q:q + 2, q:q + 2] += t[q] * np.array([[1.0, -1.0], [-1.0, 1.0]])
+    r = 1.0 / np.sqrt(S)
+    return r[:, None] * np.linalg.eigh(r[:, None] * T * r)[1], S
+
+
+def _rhs_of_modes(c, parts):
+    """the sum of amplitude x mode m x a random pattern of the columns"""
+    phi, S = _modes(c)
+    rhs = c.cell_field()
+    for m, amplitude, seed in parts:
+        f = np.random.default_rng(seed).standard_normal(c.N_CELL0)
+        rhs[:c.N_CELL0, 1:-1] += amplitude * (f - f.mean())[:, None] * (S * phi[:, m])[None, :]
+    return rhs
+
+
+def test_modal_batched_finished_mode_stays():
+    """Mode 1 ends before mode 0, which shares its group of four: its solution
+    is the one it has beside mode 4, of the next group.  One cycle (the cap
+    2 max_iters + 100 = 0), so that no later one hides a difference.  The two
+    solves round differently in their sums and in the FP32 preconditioner,
+    1e-7 of a step that is itself 2e-6 of the solution at the stop; steps
+    taken after it made 1e-5."""
+    from nsx.device import Context
+    c = make_case(160, 77, 6, seed=11, jitter=0.1)
+    phi, S = _modes(c)
+    G = Context(c)
+    G.set_params(eps=1e-6, max_iters=-50)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    G.init_state()
+    x = []
+    for other in (0, 4):
+        p, _, info = G.bicgstab(c.cell_field(), _rhs_of_modes(c, [(1, 1.0, 3), (other, 100.0, 4)]))
+        assert info["exit"] == "converged" and info["outer_passes"] == 1, info
+        x.append(interior(c, p) @ (S * phi[:, 1]))
+    G.close()
+    assert rel_err(x[0], x[1]) <= 1e-10
