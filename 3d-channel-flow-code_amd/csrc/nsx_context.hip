@@ -135,7 +135,9 @@ struct nsx_ctx {
   double *pguess = nullptr;
   int guess_stage = -1;
   // the vertical-mode solve (NSX_REFINE_MODAL): the column graph kept from
-  // nsx_commit, the device tables once built, the cycles of the last solve
+  // nsx_commit, the device tables once built, how much of the next solve is
+  // queued before its state is read (cycles; iterations of the batched form's
+  // first cycle and of the others): after what the last solve took
   std::vector<int> h_nbr;
   std::vector<double> h_ppec;
   ModalDev modal{};
@@ -1410,34 +1412,50 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
   // x = x0, r = b - A x0, the norms of b and the no-solve test
   LAUNCH(launch_bicg_init(g, s, rhs, phi_in, x, ctx->sr, r, ctx->part, ctx->st_dev, ctx->eps, ctx->MaxIters));
   LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 1, cap));
-  const size_t pend0 = ctx->pending.size();
-  // as many cycles as the last solve took, then one at a time
-  for (int cycles = std::max(2, ctx->modal_cycles), issued = 0;; cycles = 1) {
-    for (int c = 0; c < cycles; ++c, ++issued) {
+  // Queued: as many cycles as the last solve took, then one at a time; of the
+  // batched form's iterations as many as that solve's cycles took and a few
+  // more.  A batched cycle that needs more waits for the host (NSX_WAITS) and
+  // goes on where it was, so a solve's result is its own whatever was queued.
+  const SolverState &h = *ctx->st_host;
+  for (int cycle = 0, it0 = 0, cycles = std::max(2, ctx->modal_cycles);; cycles = 1) {
+    size_t kept = ctx->pending.size();
+    for (int c = 0; c < cycles; ++c) {
+      const bool on = c == 0 && it0 > 0;  // the rest of a cycle that waits
       hipEvent_t *ev = nullptr;
       if (ctx->timing) {
         ev = events(ctx, 8);
         if (!ev) return nsx_fail(ctx, -2, "hipEventCreate failed");
       }
-      LAUNCH(launch_modal_fwd(g, s, ctx->modal, r, ctx->st_dev, ev));
-      LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, issued ? ctx->modal_more : ctx->modal_iters,
-                             ev ? ev + 2 : nullptr));
+      if (on) {
+        LAUNCH(launch_modal_resume(s, ctx->st_dev));
+        LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, it0, std::max(4, it0 / 4), ev ? ev + 2 : nullptr));
+      } else {
+        LAUNCH(launch_modal_fwd(g, s, ctx->modal, r, ctx->st_dev, ev));
+        LAUNCH(launch_modal_2d(s, ctx->modal, ctx->st_dev, 0, cycle + c ? ctx->modal_more : ctx->modal_iters,
+                               ev ? ev + 2 : nullptr));
+      }
       LAUNCH(launch_modal_bwd(g, s, ctx->modal, x, ctx->st_dev, ev ? ev + 4 : nullptr));
       LAUNCH(launch_modal_true(g, s, rhs, x, r, ctx->part, ctx->st_dev, ev ? ev + 6 : nullptr));
       LAUNCH(launch_modal_check(g, s, ctx->part, ctx->st_dev, 0, cap));
       if (ev) {
         const size_t base = (size_t)(ev - &ctx->evpool[0]);
-        for (int q = 0; q < 4; ++q) ctx->pending.push_back({base + 2 * q, 16 + q});
+        for (int q = on ? 1 : 0; q < 4; ++q) ctx->pending.push_back({base + 2 * q, 16 + q});
       }
     }
     HIPCHECK(hipMemcpyAsync(ctx->st_host, ctx->st_dev, sizeof(SolverState), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
-    if (ctx->st_host->done) break;
-    if (issued > cap) return nsx_fail(ctx, -4, "solver did not stop after %d cycles", issued);
+    if (ctx->timing) {
+      // what ran: the cycles ended, and of one that waits all before its transform back
+      const int ran = h.mp_pass - cycle, first = it0 > 0 ? 3 : 4;
+      kept += ran > 0 ? first + 4 * (size_t)(ran - 1) : 0;
+      if (h.done == NSX_WAITS) kept += ran == 0 && it0 > 0 ? 1 : 2;
+      if (ctx->pending.size() > kept) ctx->pending.resize(kept);
+    }
+    if (h.done && h.done != NSX_WAITS) break;
+    cycle = h.mp_pass;
+    it0 = h.done ? h.m_wait : 0;
+    if (cycle > cap) return nsx_fail(ctx, -4, "solver did not stop after %d cycles", cycle);
   }
-  const SolverState &h = *ctx->st_host;
-  // timing: the cycles that ran
-  if (ctx->timing && ctx->pending.size() > pend0 + 4 * (size_t)h.mp_pass) ctx->pending.resize(pend0 + 4 * (size_t)h.mp_pass);
   collect_timing(ctx);
   const int it = h.m_iters;
   if (h.mp_pass > 0) {

@@ -83,6 +83,7 @@ struct SolverState {
   int m_cyc;          // most iterations of a mode in this cycle                 (2D solves; backward transform: 0)
   int m_iters;        // sum of m_cyc over the cycles                            (backward transform)
   int m_first;        // m_cyc of the first cycle                                  (backward transform)
+  int m_wait;         // iterations a batched cycle has had when its queue ended   (k_mb_final)
 };
 
 // the vectors of the single-reduction CG: e and p in place, the scaled
@@ -220,8 +221,13 @@ int launch_gnorm_sum(const Geo &g, hipStream_t s, const double *x, Partials part
 // Phi^T r), r = b - A x, the stopping rule.  ev: null, or the dispatch's start and stop
 int launch_modal_fwd(const Geo &g, hipStream_t s, const ModalDev &M, const double *r, SolverState *st,
                      hipEvent_t *ev);
-// (iters: the most iterations of the batched form)
-int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int iters, hipEvent_t *ev);
+// (The batched form queues `iters` iterations from the it0-th on; where modes
+// still iterate then and the cycle may go on, st->done = NSX_WAITS: all that is
+// queued behind returns at once, until launch_modal_resume.  So what the host
+// queues decides no result)
+#define NSX_WAITS 2
+int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int it0, int iters, hipEvent_t *ev);
+int launch_modal_resume(hipStream_t s, SolverState *st);
 int launch_modal_bwd(const Geo &g, hipStream_t s, const ModalDev &M, double *x, SolverState *st, hipEvent_t *ev);
 int launch_modal_true(const Geo &g, hipStream_t s, const double *rhs, const double *x, double *r, Partials part,
                       const SolverState *st, hipEvent_t *ev);

@@ -918,9 +918,17 @@ __global__ __launch_bounds__(T2) void k_mb_below(ModalDev M, const SolverState *
   for (int i = tid; i < A.n; i += T2) M.y2[(size_t)i * mp + m] = vget(y, i);
 }
 
-// no correction from a mode whose solve gained nothing
-__global__ __launch_bounds__(MB) void k_mb_final(ModalDev M, const SolverState *st) {
+// the queue's end after `it` iterations: wait for more, or the cycle's end (no
+// correction from a mode whose solve gained nothing)
+__global__ __launch_bounds__(MB) void k_mb_final(ModalDev M, SolverState *st, int it) {
   if (st->done) return;
+  if (it < NSX_MB_ITERS && M.nact[it] > 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      st->m_wait = it;
+      st->done = NSX_WAITS;
+    }
+    return;
+  }
   bool any = false;
   for (int m = 0; m < M.nzi; ++m) any = any || !(M.ms[m].rr <= M.ms[m].r0);
   if (!any) return;
@@ -930,15 +938,22 @@ __global__ __launch_bounds__(MB) void k_mb_final(ModalDev M, const SolverState *
   }
 }
 
-static int launch_batched(hipStream_t s, const ModalDev &M, SolverState *st, int iters) {
+__global__ void k_modal_resume(SolverState *st) {
+  if (st->done == NSX_WAITS) st->done = 0;
+}
+
+static int launch_batched(hipStream_t s, const ModalDev &M, SolverState *st, int it0, int iters) {
   const dim3 grid(NSX_MB_GRID), blk(MB), sc(M.kt);
-  hipLaunchKernelGGL(k_mb_clear, dim3(1), dim3(64), 0, s, M, st);
-  hipLaunchKernelGGL(k_mb_mean, dim3(NSX_MB_MEAN), blk, 0, s, M, st);
-  hipLaunchKernelGGL(k_mb_norm, grid, blk, 0, s, M, st);
-  hipLaunchKernelGGL(k_mb_scalars<0>, sc, dim3(T2), 0, s, M, st, 0);
-  hipLaunchKernelGGL(k_mb_update<true>, grid, blk, 0, s, M, (const float *)nullptr, st, 0);
+  if (it0 == 0) {
+    hipLaunchKernelGGL(k_mb_clear, dim3(1), dim3(64), 0, s, M, st);
+    hipLaunchKernelGGL(k_mb_mean, dim3(NSX_MB_MEAN), blk, 0, s, M, st);
+    hipLaunchKernelGGL(k_mb_norm, grid, blk, 0, s, M, st);
+    hipLaunchKernelGGL(k_mb_scalars<0>, sc, dim3(T2), 0, s, M, st, 0);
+    hipLaunchKernelGGL(k_mb_update<true>, grid, blk, 0, s, M, (const float *)nullptr, st, 0);
+  }
   const ModalLevelDev &C = M.lev[0], &A = M.lev[1];
-  for (int it = 0; it < iters && it < NSX_MB_ITERS; ++it) {
+  const int end = it0 + iters < NSX_MB_ITERS ? it0 + iters : NSX_MB_ITERS;
+  for (int it = it0; it < end; ++it) {
     hipLaunchKernelGGL(k_mb_columns<0>, grid, blk, 0, s, M, st, it);
     hipLaunchKernelGGL(k_mb_columns<1>, grid, blk, 0, s, M, st, it);
     hipLaunchKernelGGL(k_mb_restrict, grid, blk, 0, s, M, C.Rc, 1, (const float *)M.V, M.b1, M.t1, st, it);
@@ -958,7 +973,12 @@ static int launch_batched(hipStream_t s, const ModalDev &M, SolverState *st, int
     hipLaunchKernelGGL(k_mb_update<false>, grid, blk, 0, s, M, (const float *)M.P[(it + 1) & 1], st, it);
     hipLaunchKernelGGL(k_mb_scalars<3>, sc, dim3(T2), 0, s, M, st, it);
   }
-  hipLaunchKernelGGL(k_mb_final, grid, blk, 0, s, M, st);
+  hipLaunchKernelGGL(k_mb_final, grid, blk, 0, s, M, st, end);
+  return (int)hipGetLastError();
+}
+
+int launch_modal_resume(hipStream_t s, SolverState *st) {
+  hipLaunchKernelGGL(k_modal_resume, dim3(1), dim3(1), 0, s, st);
   return (int)hipGetLastError();
 }
 
@@ -967,10 +987,10 @@ int launch_modal_fwd(const Geo &g, hipStream_t s, const ModalDev &M, const doubl
   return launch_transform(g, s, M, r, nullptr, st, true, ev);
 }
 
-int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int iters, hipEvent_t *ev) {
+int launch_modal_2d(hipStream_t s, const ModalDev &M, SolverState *st, int it0, int iters, hipEvent_t *ev) {
   if (M.batched) {
     if (ev) (void)hipEventRecord(ev[0], s);
-    const int rc = launch_batched(s, M, st, iters);
+    const int rc = launch_batched(s, M, st, it0, iters);
     if (ev) (void)hipEventRecord(ev[1], s);
     return rc;
   }

@@ -151,3 +151,30 @@ def test_modal_batched_finished_mode_stays():
         x.append(interior(c, p) @ (S * phi[:, 1]))
     G.close()
     assert rel_err(x[0], x[1]) <= 1e-10
+
+
+@pytest.mark.parametrize("easy_mode", [5, 2])
+def test_modal_batched_does_not_remember(easy_mode):
+    """A batched solve gives the bits of a fresh context's whatever the context
+    solved before: an easy right-hand side (one high mode, few iterations)
+    leaves few iterations queued for the next one."""
+    from nsx.device import Context
+    c = make_case(160, 77, 6, seed=11, jitter=0.1)
+    hard = c.cell_field()
+    hard[:c.N_CELL0, 1:-1] = np.random.default_rng(8).standard_normal((c.N_CELL0, c.NZ - 2))
+    easy = _rhs_of_modes(c, [(easy_mode, 1.0, 9)])
+    out = []
+    for before in ([], [easy], [easy, easy, hard, easy]):
+        G = Context(c)
+        G.set_params(eps=EPS)
+        G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+        G.init_state()
+        its = [G.bicgstab(c.cell_field(), b)[2]["iters"] for b in before]
+        phi, pv, info = G.bicgstab(c.cell_field(), hard)
+        G.close()
+        assert info["exit"] == "converged", info
+        assert all(i < info["iters"] for i in its[:2]), (its, info)
+        out.append((phi, pv, info["iters"], info["outer_passes"], info["e1"], info["e2"]))
+    for o in out[1:]:
+        assert o[2:] == out[0][2:], (o[2:], out[0][2:])
+        assert np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
