@@ -934,23 +934,27 @@ extern "C" int nsx_get_field(nsx_ctx *ctx, int f, double *host, int fill_ghost_r
     HIPCHECK(hipEventRecord(X.done[q], s));
     return 0;
   };
+  // The crossing waits for the host's copy (and the page faults of a fresh
+  // array): large fields are copied by four threads, each taking every fourth
+  // layer of a chunk, or where a chunk has fewer than four (columns past
+  // 131,072) a quarter of each layer.  `ready` counts the chunks that have
+  // arrived (or -1: an error ended the call), `copied` the shares done.
+  const int nt = (size_t)kz * w >= NSX_XFER_THREADS ? 4 : 1, parts = step < nt ? nt : 1;
   // rows that no rule fills stay as the caller left them
   const bool whole = w == n || X.contiguous;
+  const size_t m = (size_t)(whole ? w : n);
   auto copy_rows = [&](int c, int first, int every) {
     const int k0 = c * step, nk = std::min(step, kz - k0);
-    for (int k = first; k < nk; k += every) {
+    for (int q = first; q < nk * parts; q += every) {
+      const int k = q / parts, part = q % parts;
       const double *src = X.pin[c & 1] + (size_t)k * w;
       double *dst = host + (size_t)(k0 + k) * ld;
-      memcpy(dst, src, (size_t)(whole ? w : n) * sizeof(double));
-      if (!whole)
+      const size_t a = m * part / parts, b = m * (part + 1) / parts;
+      memcpy(dst + a, src + a, (b - a) * sizeof(double));
+      if (!whole && part == 0)
         for (int e = 0; e < X.nrow; ++e) dst[X.row[e]] = src[n + e];
     }
   };
-  // The crossing waits for the host's copy (and the page faults of a fresh
-  // array): large fields are copied by four threads, each taking every fourth
-  // layer of a chunk.  `ready` counts the chunks that have arrived (or -1: an
-  // error ended the call), `copied` the shares done.
-  const int nt = step >= 4 && (size_t)kz * w >= NSX_XFER_THREADS ? 4 : 1;
   std::atomic<int> ready{0}, copied{0};
   std::vector<std::thread> team;
   struct Join {

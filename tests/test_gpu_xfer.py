@@ -22,6 +22,8 @@ pytestmark = pytest.mark.gpu
     (90, 45, 67, None),       # 4.5 MB: two chunks, the last ragged
     (128, 64, 64, (0, 0, 0, 0)),  # three chunks
     (180, 91, 67, None),      # 18 MB: several threads copy
+    (288, 229, 17, (1, 0, 0, 0)),  # 131,904 columns: three layers a chunk for four threads
+    (400, 330, 16, None),     # 264,000 columns: one layer a chunk
 ])
 def test_round_trip(nx, ny, nn, walls):
     from nsx.device import Context
