@@ -49,3 +49,17 @@ def test_round_trip(nx, ny, nn, walls):
             assert np.array_equal(out[g], a[g] if wall else a[partner[g - n0]]), (name, g)
         assert np.all(out[nex:] == -7.0), name
     G.close()
+
+
+def test_small_mesh_takes_little():
+    """The transfers' buffers follow the mesh: no megabytes on the device for
+    fields of kilobytes (the allocator's own granule is 2 MB)."""
+    from nsx.device import Context
+    c = make_case(8, 6, 6, seed=3)
+    G = Context(c)
+    before = G.device_memory_used()
+    G.put("UFN", c.u0)
+    G.get("UFN")
+    used = G.device_memory_used() - before
+    G.close()
+    assert used <= 2 << 20, used
