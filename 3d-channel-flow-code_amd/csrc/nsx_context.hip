@@ -153,7 +153,7 @@ struct nsx_ctx {
   size_t evused = 0;
   Timer t_k[3], t_stage, t_cg[2];  // FP64 A, B, C; stage kernels; FP32 CG W, X
   Timer t_cgs, t_cgs64;              // single-reduction CG, FP32 and FP64
-  Timer t_mod[5];                    // vertical-mode solve: forward transform, 2D solves, backward, true residual
+  Timer t_mod[4];                    // vertical-mode solve: forward transform, 2D solves, backward, true residual
   // (event index, timer: 0..2 FP64 solver, 5 stage, 12..13 FP32 CG, 14 single-reduction CG, 15 its FP64 instance)
   std::vector<std::pair<size_t, int>> pending;
 };
@@ -1030,10 +1030,10 @@ static hipEvent_t *events(nsx_ctx *ctx, int n) {
 static void collect_timing(nsx_ctx *ctx) {
   if (!ctx->timing) return;
   (void)hipStreamSynchronize(ctx->stream);
-  Timer *t[21] = {&ctx->t_k[0],   &ctx->t_k[1],   &ctx->t_k[2],   nullptr,        nullptr,      &ctx->t_stage,
+  Timer *t[20] = {&ctx->t_k[0],   &ctx->t_k[1],   &ctx->t_k[2],   nullptr,        nullptr,      &ctx->t_stage,
                   nullptr,         nullptr,         nullptr,         nullptr,         nullptr,      nullptr,
                   &ctx->t_cg[0],   &ctx->t_cg[1],   &ctx->t_cgs,     &ctx->t_cgs64,   &ctx->t_mod[0],
-                  &ctx->t_mod[1],  &ctx->t_mod[2],  &ctx->t_mod[3],  &ctx->t_mod[4]};
+                  &ctx->t_mod[1],  &ctx->t_mod[2],  &ctx->t_mod[3]};
   for (auto &pr : ctx->pending) {
     float ms = 0.f;
     if (t[pr.second] && hipEventElapsedTime(&ms, ctx->evpool[pr.first], ctx->evpool[pr.first + 1]) == hipSuccess) {
@@ -2759,8 +2759,8 @@ extern "C" int nsx_timing_get(nsx_ctx *ctx, const char *name, double *total_ms, 
     if (!strcmp(name, names_cg[q])) t = &ctx->t_cg[q];
   if (!strcmp(name, "cg32_sr")) t = &ctx->t_cgs;
   if (!strcmp(name, "cg64_sr")) t = &ctx->t_cgs64;
-  static const char *names_mod[5] = {"modal_fwd", "modal_mg", "modal_bwd", "modal_spmv", "modal_update"};
-  for (int q = 0; q < 5; ++q)
+  static const char *names_mod[4] = {"modal_fwd", "modal_mg", "modal_bwd", "modal_spmv"};
+  for (int q = 0; q < 4; ++q)
     if (!strcmp(name, names_mod[q])) t = &ctx->t_mod[q];
   if (!t) return nsx_fail(ctx, -1, "unknown timer %s", name);
   if (total_ms) *total_ms = t->ms;
@@ -2772,6 +2772,6 @@ extern "C" int nsx_timing_reset(nsx_ctx *ctx) {
   if (!ctx) return -1;
   for (int q = 0; q < 3; ++q) ctx->t_k[q] = Timer{};
   ctx->t_stage = ctx->t_cg[0] = ctx->t_cg[1] = ctx->t_cgs = ctx->t_cgs64 = Timer{};
-  for (int q = 0; q < 5; ++q) ctx->t_mod[q] = Timer{};
+  for (int q = 0; q < 4; ++q) ctx->t_mod[q] = Timer{};
   return 0;
 }
