@@ -1255,7 +1255,8 @@ static int modal_setup(nsx_ctx *ctx) {
   if (ctx->modal_ok) return 0;
   const int N0 = ctx->N0, NZ = ctx->NZ, nzi = NZ - 2;
   // vertical couplings per unit area between interior layers k and k+1,
-  // 1/dsig(k) (the quotient area/dsig(k) of the rows)
+  // 1/dsig(k) (the quotient area/dsig(k) of the rows); none at the ends: the
+  // products mirror the end layers whatever bctop and bcbot are (apply_row)
   std::vector<double> tlay((size_t)nzi, 0.0), svl((size_t)nzi);
   for (int k = 1; k <= NZ - 3; ++k) tlay[k - 1] = 1.0 / ctx->dsig[k];
   for (int k = 1; k <= NZ - 2; ++k) svl[k - 1] = ctx->dsigv[k - 1];

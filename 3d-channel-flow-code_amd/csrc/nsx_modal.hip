@@ -4,17 +4,17 @@
 // The PPE operator of the prismatic sigma grid is a Kronecker sum: a
 // horizontal coupling between columns i and j at layer k is ppec(i,j)
 // dsigv(k-1), a vertical one between layers k and k+1 of column i is area(i)
-// t(k) (t = 1/dsig, none at the top and bottom, whose ghosts are Neumann), and the diagonal
-// closes every row to zero (PDE_center, PDE.F90:8-135).  So -A = L (x) S +
-// D (x) T with L the weighted graph Laplacian of the columns, D = diag(area),
-// S = diag(dsigv) and T the layers' 1D Laplacian.  The generalized
-// eigenvectors Phi of (T, S) (Phi^T S Phi = I, Phi^T T Phi = diag(mu)) split
-// -A y = r into one 2D problem per vertical mode m, (L + mu_m D) yh_m =
-// (Phi^T r)_m with y = Phi yh.  The solve transforms a residual once, solves
-// every mode's 2D problem by conjugate gradients of its own, and transforms
-// back; the 2D preconditioner is a V-cycle of smoothed-aggregation multigrid
-// on the column graph.  This file builds the tables on the host: the modes,
-// the hierarchy, the coarsest level's inverses.  The kernels are in
+// t(k) (t = 1/dsig, none at the top and bottom, which every product mirrors),
+// and the diagonal closes every row to zero (PDE_center, PDE.F90:8-135).  So
+// -A = L (x) S + D (x) T with L the weighted graph Laplacian of the columns, D
+// = diag(area), S = diag(dsigv) and T the layers' 1D Laplacian.  The
+// generalized eigenvectors Phi of (T, S) (Phi^T S Phi = I, Phi^T T Phi =
+// diag(mu)) split -A y = r into one 2D problem per vertical mode m, (L + mu_m
+// D) yh_m = (Phi^T r)_m with y = Phi yh.  The solve transforms a residual
+// once, solves every mode's 2D problem by conjugate gradients of its own, and
+// transforms back; the 2D preconditioner is a V-cycle of smoothed-aggregation
+// multigrid on the column graph.  This file builds the tables on the host: the
+// modes, the hierarchy, the coarsest level's inverses.  The kernels are in
 // nsx_modal_dev.hip.
 //
 // The hierarchy is built from L alone and serves every mode: aggregates are a

@@ -1,8 +1,7 @@
-"""The precision form's CG preconditioned by the vertical modes of the
-operator (NSX_REFINE_MODAL): per column the generalized eigenvectors of the
-vertical couplings split A into one 2D problem per mode, the 16 lowest go
-through a V-cycle of aggregation multigrid on the column graph, the others
-are scaled by their diagonal.
+"""The vertical-mode pressure solve (NSX_REFINE_MODAL): per column the
+generalized eigenvectors of the vertical couplings split A into one 2D
+problem per mode, each solved by FP64 CG with an FP32 multigrid, in cycles
+from the true FP64 residual.
 
   * random right-hand sides on the 32x16 quads x 32 layers channel and the
     walled duct: the solve meets the reference's stopping rule on its true
@@ -10,12 +9,10 @@ are scaled by their diagonal.
     eps for the summation order) and agrees with the FP64 BiCGSTAB and the
     oracle to 1e-6 (both stop at 1e-10 of an operator with condition number
     O(1e4));
-  * a 24x16 quads x 140 layers channel, whose columns hold more slots than
-    the matrix-core transforms take (128): the vector-unit transforms, same
-    checks against the FP64 BiCGSTAB;
-  * an 8x6 quads x 6 layers channel with a bed: fewer layers than the
-    multigrid's 16 modes (all 6 go through it), a single level (the dense
-    coarse solve on the 96 columns), one mode tile of the transforms; a
+  * a 24x16 quads x 140 layers channel, whose transforms' table takes two
+    panels: same checks against the FP64 BiCGSTAB;
+  * an 8x6 quads x 6 layers channel with a bed: a single level (the dense
+    coarse solve on the 96 columns), one tile of the transforms; a
     stage of nsx_hydro in the precision form against the FP64 path;
   * the 64x32 quads x 48 layers channel: a random right-hand side solved to
     eps 1e-13 in a fraction of the block-Jacobi instance's iterations, and
@@ -51,7 +48,7 @@ def _solve_pair(c, seed):
 def test_modal_solve_random_rhs(seed):
     c = config_case(0, jitter=0.1)
     rhs, phi0, (phi64, pv64, _), (phim, pvm, im) = _solve_pair(c, seed)
-    print(f"modal CG: {im['iters']} iterations, {im['outer_passes']} true residuals", flush=True)
+    print(f"modal solve: {im['iters']} iterations, {im['outer_passes']} true residuals", flush=True)
     assert im["exit"] == "converged" and im["iters_fp32"] > 0, im
     assert min(im["e1"], im["e2"]) < c.params.eps
     e1, e2 = ppe_residual(c, phim, rhs)
@@ -77,7 +74,7 @@ def test_modal_solve_tall_columns():
     c = make_case(24, 16, 140, jitter=0.1)
     assert c.NZ > 130
     rhs, _, (phi64, pv64, _), (phim, pvm, im) = _solve_pair(c, 8)
-    print(f"modal CG, {c.NZ} layers: {im['iters']} iterations", flush=True)
+    print(f"modal solve, {c.NZ} layers: {im['iters']} iterations", flush=True)
     assert im["exit"] == "converged" and im["iters_fp32"] > 0, im
     e1, e2 = ppe_residual(c, phim, rhs)
     assert min(e1, e2) < 2 * c.params.eps, (e1, e2)

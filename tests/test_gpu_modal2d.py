@@ -46,9 +46,10 @@ def _check(c, seed):
     (13, 9, 17),     # one layer past a tile, odd columns
     (40, 21, 33),    # 1,680 columns, three levels
     (12, 8, 130),    # two panels
-    (12, 8, 260),    # seventeen tiles, one past the eight a block accumulates twice over
-    (90, 41, 9),     # 7,380 columns: the columns' vectors pass the block's LDS
-    (160, 76, 6),    # 24,320 columns: the most that take a block per mode
+    (12, 8, 260),    # seventeen tiles: panels of the four that fit the LDS, the last with one
+    (90, 41, 9),     # 7,380 columns: four levels, every vector in the block's LDS
+    (110, 51, 6),    # 11,220 columns: two of the columns' four vectors in LDS
+    (160, 76, 6),    # 24,320 columns, near the most that take a block per mode: none
     (160, 77, 6),    # 24,640: batched over the modes, ten of a tile's sixteen unused
     (201, 79, 17),   # odd columns, one mode past a tile
     (160, 80, 67),   # five tiles: thread groups that do not divide a block
@@ -109,6 +110,35 @@ def test_modal_deep_columns(nn):
     assert min(e1, e2) < 2e-8, (e1, e2)
 
 
+@pytest.mark.parametrize("bctop, bcbot", [(0, 1), (0, 0)])
+@pytest.mark.parametrize("nx, ny, nn", [(40, 21, 33), (160, 77, 6)])
+def test_modal_open_ends(nx, ny, nn, bctop, bcbot):
+    """bctop or bcbot other than 1 leaves the end's coupling in the matrix, but
+    every product mirrors the end layers, as get_Apk does: the operator stays
+    the Neumann one that the modes are of, and two cycles solve it."""
+    from nsx.device import Context
+    c = make_case(nx, ny, nn, seed=6, jitter=0.1)
+    c.bctop, c.bcbot = bctop, bcbot
+    A, area = c.arrays, c.areaCell[:c.N_CELL0]
+    if not bctop:
+        A["AmCT"][:, -2] = area / c.dsig[-2]
+    if not bcbot:
+        A["AmCB"][:, 1] = area / c.dsig[0]
+    A["AmC0"][:, 1:-1] = -1.0 * (A["AmCT"] + A["AmCB"] + A["AmC1"] + A["AmC2"] + A["AmC3"])[:, 1:-1]
+    rhs = c.cell_field()
+    rhs[:c.N_CELL0, 1:-1] = np.random.default_rng(nn).standard_normal((c.N_CELL0, c.NZ - 2))
+    G = Context(c)
+    G.set_params(eps=EPS)
+    G.init_state()
+    phi64, _, _ = G.bicgstab(c.cell_field(), rhs)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    phi, _, info = G.bicgstab(c.cell_field(), rhs)
+    G.close()
+    assert info["exit"] == "converged" and info["iters_fp32"] == info["iters"] > 0, info
+    assert info["outer_passes"] == 2 and min(info["e1"], info["e2"]) < EPS, info
+    assert rel_err(interior(c, phi), interior(c, phi64)) <= 1e-6
+
+
 def _modes(c):
     """the vertical modes, columns of (NZ-2) x (NZ-2), and the layers' S"""
     n = c.NZ - 2
@@ -128,29 +158,6 @@ def _rhs_of_modes(c, parts):
         f = np.random.default_rng(seed).standard_normal(c.N_CELL0)
         rhs[:c.N_CELL0, 1:-1] += amplitude * (f - f.mean())[:, None] * (S * phi[:, m])[None, :]
     return rhs
-
-
-def test_modal_batched_finished_mode_stays():
-    """Mode 1 ends before mode 0, which shares its group of four: its solution
-    is the one it has beside mode 4, of the next group.  One cycle (the cap
-    2 max_iters + 100 = 0), so that no later one hides a difference.  The two
-    solves round differently in their sums and in the FP32 preconditioner,
-    1e-7 of a step that is itself 2e-6 of the solution at the stop; steps
-    taken after it made 1e-5."""
-    from nsx.device import Context
-    c = make_case(160, 77, 6, seed=11, jitter=0.1)
-    phi, S = _modes(c)
-    G = Context(c)
-    G.set_params(eps=1e-6, max_iters=-50)
-    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
-    G.init_state()
-    x = []
-    for other in (0, 4):
-        p, _, info = G.bicgstab(c.cell_field(), _rhs_of_modes(c, [(1, 1.0, 3), (other, 100.0, 4)]))
-        assert info["exit"] == "converged" and info["outer_passes"] == 1, info
-        x.append(interior(c, p) @ (S * phi[:, 1]))
-    G.close()
-    assert rel_err(x[0], x[1]) <= 1e-10
 
 
 @pytest.mark.parametrize("easy_mode", [5, 2])
@@ -178,3 +185,47 @@ def test_modal_batched_does_not_remember(easy_mode):
     for o in out[1:]:
         assert o[2:] == out[0][2:], (o[2:], out[0][2:])
         assert np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
+
+
+def test_modal_batched_finished_mode_stays():
+    """Mode 1 ends before mode 0, which shares its group of four: its solution
+    is the one it has beside mode 4, of the next group.  One cycle (the cap
+    2 max_iters + 100 = 0), so that no later one hides a difference.  The two
+    solves round differently in their sums and in the FP32 preconditioner,
+    1e-7 of a step that is itself 2e-6 of the solution at the stop; steps
+    taken after it made 1e-5."""
+    from nsx.device import Context
+    c = make_case(160, 77, 6, seed=11, jitter=0.1)
+    phi, S = _modes(c)
+    G = Context(c)
+    G.set_params(eps=1e-6, max_iters=-50)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    G.init_state()
+    x = []
+    for other in (0, 4):
+        p, _, info = G.bicgstab(c.cell_field(), _rhs_of_modes(c, [(1, 1.0, 3), (other, 100.0, 4)]))
+        assert info["exit"] == "converged" and info["outer_passes"] == 1, info
+        x.append(interior(c, p) @ (S * phi[:, 1]))
+    G.close()
+    assert rel_err(x[0], x[1]) <= 1e-10
+
+
+def test_modal_contexts_of_two_sizes():
+    """A small mesh's tables, made after a large one's, leave the large one's
+    solves as they were (the kernels' LDS limits belong to the process)."""
+    from nsx.device import Context
+    cases = [make_case(90, 41, 9, seed=11, jitter=0.1), make_case(2, 2, 2, seed=11, jitter=0.1)]
+    ctx, rhs, first = [], [], []
+    for c in cases:
+        G = Context(c)
+        G.set_params(eps=EPS)
+        G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+        G.init_state()
+        r = c.cell_field()
+        r[:c.N_CELL0, 1:-1] = np.random.default_rng(c.nx).standard_normal((c.N_CELL0, c.NZ - 2))
+        ctx.append(G)
+        rhs.append(r)
+        first.append(G.bicgstab(c.cell_field(), r)[0])
+    for G, c, r, phi in zip(ctx, cases, rhs, first):
+        assert np.array_equal(G.bicgstab(c.cell_field(), r)[0], phi)
+        G.close()
