@@ -347,19 +347,13 @@ int modal_build_host(int N0, int nzi, const int *nbr, const double *ppec, const 
       const int n = nbr[i * 3 + j];
       H.nb[(size_t)i * 3 + j] = i;
       if (n < 0 || n >= N0 || n == i) continue;
-      // the neighbour's weights back towards i, shared by its edges to i
+      // the neighbour's weights back towards i, shared by i's edges to it (the
+      // sums over a pair's edges agree both ways, whatever their numbers)
       double back = 0.0;
-      int to = 0, from = 0;
+      int to = 0;
       for (int q = 0; q < 3; ++q) {
-        if (nbr[n * 3 + q] == i) {
-          back += ppec[n * 3 + q];
-          ++from;
-        }
+        if (nbr[n * 3 + q] == i) back += ppec[n * 3 + q];
         if (nbr[i * 3 + q] == n) ++to;
-      }
-      if (from != to) {
-        err = "vertical-mode solve: the column graph is not symmetric";
-        return -1;
       }
       const double w = 0.5 * (ppec[i * 3 + j] + back / to);
       H.nb[(size_t)i * 3 + j] = n;

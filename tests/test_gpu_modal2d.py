@@ -229,3 +229,29 @@ def test_modal_contexts_of_two_sizes():
     for G, c, r, phi in zip(ctx, cases, rhs, first):
         assert np.array_equal(G.bicgstab(c.cell_field(), r)[0], phi)
         G.close()
+
+
+def test_modal_uneven_edges():
+    """A mesh that nsx_commit takes: one cell lists a neighbour by two edges and
+    is listed by one.  Its matrix is not symmetric and no solver converges;
+    the solve ends as the FP64 one does, with a code and not with an error."""
+    from nsx.device import Context
+    c = make_case(13, 9, 6, seed=5, jitter=0.1, walls=(1, 0, 0, 0))
+    A, cp, n0 = c.arrays, c.No_cp, c.N_CELL0
+    i = next(q for q in range(n0 // 2, n0) if np.all(cp[q] <= n0) and np.all(cp[cp[q] - 1] <= n0))
+    m = cp[i, 1] - 1
+    f = list(cp[m]).index(i + 1)
+    cp[i, 1] = cp[i, 0]
+    cp[m, f] = next(g for g in cp[:n0].ravel() if g > n0 and c.bcpc[g - 1] == 1)
+    A[f"AmC{f + 1}"][m] = 0.0
+    A["AmC0"][m, 1:-1] = -1.0 * (A["AmCT"] + A["AmCB"] + A["AmC1"] + A["AmC2"] + A["AmC3"])[m, 1:-1]
+    rhs = c.cell_field()
+    rhs[:n0, 1:-1] = np.random.default_rng(1).standard_normal((n0, c.NZ - 2))
+    G = Context(c)
+    G.set_params(max_iters=50)
+    G.init_state()
+    _, _, i64 = G.bicgstab(c.cell_field(), rhs)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    _, _, info = G.bicgstab(c.cell_field(), rhs)
+    G.close()
+    assert info["exit"] == i64["exit"] == "max iterations", (info, i64)
