@@ -280,6 +280,7 @@ __global__ __launch_bounds__(NSX_BLOCK) void k_bicg_init_state(SolverState *st, 
     st->m_cyc = 0;
     st->m_first = 0;
     st->m_stall = 0;
+    st->m_swept = 0;
     st->delta = delta;
     st->ureq[0] = st->ureq[1] = 0;
   }

@@ -153,6 +153,7 @@ struct nsx_ctx {
   size_t evused = 0;
   Timer t_k[3], t_stage, t_cg[2];  // FP64 A, B, C; stage kernels; FP32 CG W, X
   Timer t_cgs, t_cgs64;              // single-reduction CG, FP32 and FP64
+  Timer t_swept;                     // (no time) modes swept by its 2D solves, summed over their iterations
   Timer t_mod[4];                    // vertical-mode solve: forward transform, 2D solves, backward, true residual
   // (event index, timer: 0..2 FP64 solver, 5 stage, 12..13 FP32 CG, 14 single-reduction CG, 15 its FP64 instance)
   std::vector<std::pair<size_t, int>> pending;
@@ -1468,6 +1469,7 @@ static int solve_modal(nsx_ctx *ctx, const double *rhs, const double *phi_in, do
     it0 = h.done ? h.m_wait : 0;
     if (cycle > cap) return nsx_fail(ctx, -4, "solver did not stop after %d cycles", cycle);
   }
+  if (ctx->timing) ctx->t_swept.n += h.m_swept;
   collect_timing(ctx);
   const int it = h.m_iters;
   if (h.mp_pass > 0) {
@@ -2760,6 +2762,7 @@ extern "C" int nsx_timing_get(nsx_ctx *ctx, const char *name, double *total_ms, 
     if (!strcmp(name, names_cg[q])) t = &ctx->t_cg[q];
   if (!strcmp(name, "cg32_sr")) t = &ctx->t_cgs;
   if (!strcmp(name, "cg64_sr")) t = &ctx->t_cgs64;
+  if (!strcmp(name, "modal_swept")) t = &ctx->t_swept;
   static const char *names_mod[4] = {"modal_fwd", "modal_mg", "modal_bwd", "modal_spmv"};
   for (int q = 0; q < 4; ++q)
     if (!strcmp(name, names_mod[q])) t = &ctx->t_mod[q];
@@ -2772,7 +2775,7 @@ extern "C" int nsx_timing_get(nsx_ctx *ctx, const char *name, double *total_ms, 
 extern "C" int nsx_timing_reset(nsx_ctx *ctx) {
   if (!ctx) return -1;
   for (int q = 0; q < 3; ++q) ctx->t_k[q] = Timer{};
-  ctx->t_stage = ctx->t_cg[0] = ctx->t_cg[1] = ctx->t_cgs = ctx->t_cgs64 = Timer{};
+  ctx->t_stage = ctx->t_cg[0] = ctx->t_cg[1] = ctx->t_cgs = ctx->t_cgs64 = ctx->t_swept = Timer{};
   for (int q = 0; q < 4; ++q) ctx->t_mod[q] = Timer{};
   return 0;
 }

@@ -83,6 +83,7 @@ struct SolverState {
   int m_cyc;          // most iterations of a mode in this cycle                 (2D solves; backward transform: 0)
   int m_iters;        // sum of m_cyc over the cycles                            (backward transform)
   int m_first;        // m_cyc of the first cycle                                  (backward transform)
+  int m_swept;        // modes swept, summed over the iterations                  (2D solves)
   int m_wait;         // iterations a batched cycle has had when its queue ended   (k_mb_final)
 };
 

@@ -490,7 +490,10 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
   // no correction from a solve that gained nothing
   if (!(rr < r0))
     for (int i = tid; i < N0; i += T2) x[i] = 0.0;
-  if (tid == 0) atomicMax(&st->m_cyc, it);
+  if (tid == 0) {
+    atomicMax(&st->m_cyc, it);
+    atomicAdd(&st->m_swept, it);
+  }
 }
 
 // --- the 2D solves batched over the modes, for meshes whose vectors pass the
@@ -651,7 +654,10 @@ __global__ __launch_bounds__(T2) void k_mb_scalars(ModalDev M, SolverState *st, 
       S.as = 0.0;
       S.beta = 0.f;
     }
-    if (m == 0) st->m_cyc = it + 1;
+    if (m == 0) {
+      st->m_cyc = it + 1;
+      st->m_swept += cur;
+    }
   }
 }
 
