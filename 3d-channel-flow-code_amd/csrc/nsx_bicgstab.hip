@@ -748,11 +748,10 @@ __global__ __launch_bounds__(NSX_BLOCK) void k_bicg_c(Geo g, T *x, T *rt, T *q, 
 // other.  Here every load (the partial sums, the levels, the neighbours, the
 // vectors at the window and at its outer neighbours) is issued before the
 // first barrier, which the reduction and the level table share.  The values
-// formed are those of the swept kernels.  A and B, us, before -> after: 36
-// windows 10.9 -> 6.9 and 8.1 -> 5.4 (the grid of 32 blocks took two rounds),
-// 208 windows 8.9 -> 8.0 and 6.5 -> 5.6, 352 windows 10.8 -> 9.1 and 7.4 ->
-// 6.4; at 1,088 windows the swept ones win (the blocks no longer wait alone).
-// Phase C the same way gained nothing (208 windows: 6.6 -> 7.4).
+// formed are those of the swept kernels.  A whole iteration takes 19.0 us
+// against 20.6 of the swept form on 10 windows, 20.3 against 21.7 on 36 and 21.5
+// against 21.9 on 144; from 176 the swept form is the faster (NSX_ONE_WINDOW).
+// Phase C the same way gained nothing.
 template <int K>
 __device__ inline void part_load(const double *P, double (&v)[K]) {
 #pragma unroll

@@ -62,9 +62,11 @@ struct Xfer {
 };
 // 4 MB: a chunk's crossing (70 us) hides its launches, two stay in the host's cache
 #define NSX_XFER_CHUNK (512 * 1024)
-// up to so many values the host transposes (a kernel's launch costs more: at 6,528
-// values a stage's 18 transfers took 100 us longer with it; at 36,864 it saves 30 %
-// of the single routines' calls)
+// Up to so many values the host transposes instead of a kernel.  Put and get,
+// host against kernel, us: 4,096 values 12.7 and 13.2 against 16.9 and 17.6;
+// 8,192 13.0 and 18.8 against 17.0 and 18.7; 10,752 13.9 and 21.5 against
+// 17.1 and 19.5; 16,384 15.9 and 26.8 against 17.7 and 21.4; 32,768 23.2 and
+// 46.2 against 23.2 and 34.2.  A put and a get together cross near 12,000
 #define NSX_XFER_HOST 16384
 // values from which four threads copy (16 MB)
 #define NSX_XFER_THREADS (2 * 1024 * 1024)

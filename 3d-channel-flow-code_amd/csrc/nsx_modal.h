@@ -15,10 +15,18 @@
 #define NSX_MODAL_OMEGA 0.8f
 #define NSX_MODAL_POMEGA (2.0 / 3.0)
 // Columns from which the 2D solves run batched over the modes (one launch per
-// sweep over the chip) instead of one block per mode.  A random right-hand
-// side to 1e-13, block per mode against batched, 48 layers: 4,096 columns
-// 0.95 ms against 3.7, 8,192 2.5 against 6.0, 16,384 4.8 against 6.7; 65,536 x 96 layers 13
-// against 7.  16 layers: 16,384 columns 4.5 against 6.1.
+// sweep over the chip) instead of one block per mode.  The 2D solves of a
+// random right-hand side to 1e-13 (two cycles), block per mode against batched, ms:
+//   columns     16 layers       48           96           128
+//    8,192     2.2 / 4.2    2.3 / 4.7    2.5 / 4.8    2.5 / 4.8
+//   16,384     4.4 / 4.9    4.5 / 5.5    4.4 / 5.7    4.7 / 5.7
+//   24,576     7.6 / 5.3    7.7 / 6.5    7.7 / 6.5    8.1 / 6.8
+//   32,640     9.8 / 5.8    9.7 / 6.9    9.7 / 7.4   10.1 / 7.7
+//   65,536    19.8 / 6.8   19.7 / 8.8   20.3 / 10.7  22.4 / 11.4
+// A block's time goes with the columns, whatever the number of blocks up to
+// 128; the batched form's hardly with the columns (launches).  They cross
+// near 18,000 columns at 16 layers and 20,000 to 20,500 at 48 to 128: the line
+// lies above them all.
 #define NSX_MODAL_BATCH 24576
 // blocks of the batched kernels, and the most iterations of a cycle
 #define NSX_MB_GRID 1024
