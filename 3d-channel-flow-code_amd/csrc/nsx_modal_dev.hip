@@ -501,14 +501,15 @@ __global__ __launch_bounds__(T2) void k_modal_2d(ModalDev M, SolverState *st) {
 // launch per sweep over the chip: a thread holds four modes of a node, so the
 // graph's indices and weights are read once for all modes (one block per mode
 // reads them per mode, and is bound by its CU's address unit: 500 us an
-// iteration at 65,536 columns x 96 layers, against 190 on average here).  The columns' smoother is
+// iteration at 65,536 columns x 96 layers, against about 300 on average here).  The columns' smoother is
 // the Chebyshev one too, on the mode's own bounds: the high modes, most of the
 // work, take 6 to 11 iterations for 1e-10 instead of 11 to 17, for two more sweeps.
 // Levels 2 and below run one block per mode in LDS.  Modes whose residual has
 // met its target stop; the rows are swept up to the last mode still
 // iterating.  At 6.3M prisms with all modes iterating the update moves 350 MB
-// in 75 us (4.6 TB/s) and the product 126 MB and its gathers in 46 us; with few modes the 18
-// launches' latency bounds the iteration.
+// in 75 us (4.6 TB/s) and the product 126 MB and its gathers in 46 us.  On
+// average 34 modes are swept, at 1.09 TB/s of the columns' vectors: 18 kernels of
+// 5 to 40 us, a tenth of the time between them.
 constexpr int MB = NSX_BLOCK;
 
 // f(node, q, K) over the nodes and the groups q of four modes below nact; a
