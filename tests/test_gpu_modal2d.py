@@ -187,6 +187,33 @@ def test_modal_batched_does_not_remember(easy_mode):
         assert np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
 
 
+def test_modal_batched_timers_count_what_ran():
+    """Of a solve that waits for more iterations the timers hold the cycles that
+    ran, its 2D solves in two parts or more."""
+    from nsx.device import Context
+    c = make_case(160, 77, 6, seed=11, jitter=0.1)
+    hard = c.cell_field()
+    hard[:c.N_CELL0, 1:-1] = np.random.default_rng(8).standard_normal((c.N_CELL0, c.NZ - 2))
+    G = Context(c)
+    G.set_params(eps=EPS)
+    G.set_precision(PREC_MIXED, REFINE_MODAL, 0.1, 30)
+    G.init_state()
+    G.bicgstab(c.cell_field(), _rhs_of_modes(c, [(5, 1.0, 9)]))
+    G.timing(True)
+    counts, swept = [], []
+    for _ in range(2):
+        G.timing_reset()
+        info = G.bicgstab(c.cell_field(), hard)[2]
+        for name in ("modal_fwd", "modal_bwd", "modal_spmv"):
+            ms, n = G.timer(name)
+            assert n == info["outer_passes"] and ms > 0, (name, n, info)
+        counts.append(G.timer("modal_mg")[1])
+        swept.append(G.timer("modal_swept")[1])
+    G.close()
+    assert counts[0] > counts[1] == info["outer_passes"], counts
+    assert swept[0] == swept[1] >= info["iters"], swept
+
+
 def test_modal_batched_finished_mode_stays():
     """Mode 1 ends before mode 0, which shares its group of four: its solution
     is the one it has beside mode 4, of the next group.  One cycle (the cap
